@@ -24,12 +24,14 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 namespace yabt {
 namespace bin {
 
 constexpr int SB = 1024;            // sort block
-constexpr int HT = 16;              // features per histogram / transform tile
-constexpr int TB = 256;             // threads per transform / select block
+constexpr int HT = 16;              // features per histogram tile
+constexpr int TB = 256;             // threads per select block
 constexpr int MAXE = 255;           // edges per feature (max_bins - 1 <= 255)
 
 __device__ __forceinline__ uint32_t fkey(float v) {
@@ -394,54 +396,152 @@ __global__ void k_select_finish(const uint32_t* __restrict__ cnt, int F, const u
 // transform
 // ---------------------------------------------------------------------------
 
-// One thread per (row, 16-feature tile): impute, count edges below x (binary
-// search in LDS), write the row's 16 bins to the row-major layout with one
-// 16-byte store, each bin to the feature-major layout, and the imputed value.
-__global__ void __launch_bounds__(TB) k_transform(const float* __restrict__ X, int64_t ldx, int64_t n, int F,
-                                                  const float* __restrict__ edges, int64_t ld_edges,
-                                                  const int32_t* __restrict__ nedges, const float* __restrict__ medians,
-                                                  uint8_t* __restrict__ out_fm, int64_t ld_fm,
-                                                  uint8_t* __restrict__ out_rm, int64_t ld_rm,
-                                                  float* __restrict__ out_imp, int64_t ld_imp, int rm_vec) {
-    __shared__ float s_e[HT][MAXE + 1];
-    __shared__ int s_n[HT];
-    __shared__ float s_med[HT];
-    const int f0 = blockIdx.y * HT;
-    for (int i = threadIdx.x; i < HT * (MAXE + 1); i += TB) {
-        const int j = i / (MAXE + 1), k = i % (MAXE + 1);
-        s_e[j][k] = (f0 + j < F && k < MAXE) ? edges[(size_t)(f0 + j) * ld_edges + k] : 0.0f;
-    }
-    if (threadIdx.x < HT) {
-        const int f = f0 + threadIdx.x;
-        s_n[threadIdx.x] = f < F ? min(max(nedges[f], 0), MAXE) : 0;
-        s_med[threadIdx.x] = f < F ? medians[f] : 0.0f;
+// A block keeps its feature group's edges in LDS and takes tiles of TR rows:
+//   * a tile's values are read in memory order (lanes over neighbouring
+//     features), imputed and stored the same way, and each looked up by its lane
+//     in its own feature's edges.  The edges lie as a complete search tree
+//     in level order (node k's children 2k and 2k + 1; +inf where a feature
+//     has fewer edges), so a lookup is one read, compare and add a level, as
+//     many levels as the group's longest edge list needs; tables of different
+//     features start a bank apart;
+//   * the bins wait in LDS as [feature][row] bytes and leave as 16 rows of a
+//     feature (feature-major) and as 4 x 4 blocks turned into 4 features of a
+//     row (row-major), both in whole lines.
+// Bound by HBM (X in, two byte layouts and the imputed matrix out: 1.03 GB at
+// 2M x 50) and the lookups' LDS reads: 2684 -> 365 us there (2.8 TB/s).  A row
+// per thread, as before, read X at the row stride and searched sorted edges
+// at addresses that share four of the 64 banks.
+constexpr int TT = 512;                        // threads of a transform block
+constexpr int TR = 256;                        // rows per tile
+constexpr int TSTRIDE = NB + 1;                // words between two features' tables
+constexpr int TBYTES = TR + 4;                 // bytes between two features' bins
+constexpr int TFEAT = 60;                      // features per block: two blocks' LDS on a CU
+
+struct TransformArgs {
+    const float* X;
+    int64_t ldx, n;
+    int F, fg;                                 // fg: features per group (a multiple of 4)
+    const float* edges;
+    int64_t ld_edges;
+    const int32_t* nedges;
+    const float* medians;
+    uint8_t* fm;
+    int64_t ld_fm;
+    uint8_t* rm;
+    int64_t ld_rm;
+    float* imp;
+    int64_t ld_imp;
+    int fm_vec, rm_vec;                        // 16-byte aligned layouts
+};
+
+__global__ void __launch_bounds__(TT) k_transform(TransformArgs A) {
+    extern __shared__ char smem[];
+    __shared__ int s_levels;
+    float* s_e = reinterpret_cast<float*>(smem);                       // [fg][TSTRIDE]
+    float* s_med = s_e + A.fg * TSTRIDE;                               // [fg]
+    uint8_t* s_b = reinterpret_cast<uint8_t*>(s_med + A.fg);           // [fg][TBYTES]
+    const int f0 = blockIdx.y * A.fg, nf = min(A.fg, A.F - f0);
+    const int tid = threadIdx.x;
+    if (tid == 0) s_levels = 0;
+    __syncthreads();
+    for (int j = tid; j < nf; j += TT) {
+        const int ne = min(max(A.nedges[f0 + j], 0), MAXE);
+        atomicMax(&s_levels, ne ? 32 - __clz(ne) : 0);
+        s_med[j] = A.medians[f0 + j];
     }
     __syncthreads();
-    for (int64_t r = (int64_t)blockIdx.x * TB + threadIdx.x; r < n; r += (int64_t)gridDim.x * TB) {
-        uint32_t w4[4] = {0u, 0u, 0u, 0u};
+    const int levels = s_levels, nodes = 1 << levels;
+    for (int i = tid; i < nf * nodes; i += TT) {
+        const int j = i >> levels, k = i & (nodes - 1);
+        if (k == 0) continue;
+        const int lv = 31 - __clz(k);                                  // node k: number k - 2^lv of level lv
+        const int at = ((2 * (k - (1 << lv)) + 1) << (levels - 1 - lv)) - 1;
+        const int ne = min(max(A.nedges[f0 + j], 0), MAXE);
+        s_e[j * TSTRIDE + k] = at < ne ? A.edges[(size_t)(f0 + j) * A.ld_edges + at] : INFINITY;
+    }
+    // the bins of the row-major layout's columns up to the next multiple of 16 are zero
+    const int last = blockIdx.y + 1 == gridDim.y;
+    const int nq = last && A.rm_vec ? (((A.F + 15) & ~15) - f0) / 4 : (nf + 3) / 4;
+    for (int64_t r0 = (int64_t)blockIdx.x * TR; r0 < A.n; r0 += (int64_t)gridDim.x * TR) {
+        const int rows = (int)min((int64_t)TR, A.n - r0);
+        __syncthreads();                       // the tables; the last tile's bins are out
+        const int total = rows * nf, dj = TT % nf, dr = TT / nf;
+        constexpr int U = 4;
+        int j = tid % nf, r = tid / nf;
+        for (int i0 = tid; i0 < total; i0 += TT * U) {
+            float x[U];
+            int jj[U], rr[U];
 #pragma unroll
-        for (int j = 0; j < HT; ++j) {
-            const int f = f0 + j;
-            if (f >= F) break;
-            float x = X[(size_t)r * ldx + f];
-            if (isnan(x)) x = s_med[j];
-            int lo = 0, hi = s_n[j];
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (s_e[j][mid] < x) lo = mid + 1;
-                else hi = mid;
+            for (int u = 0; u < U; ++u) {
+                jj[u] = j;
+                rr[u] = r;
+                const bool ok = i0 + u * TT < total;
+                x[u] = ok ? A.X[(size_t)(r0 + r) * A.ldx + f0 + j] : 0.0f;
+                j += dj;
+                r += dr;
+                if (j >= nf) {
+                    j -= nf;
+                    ++r;
+                }
             }
-            const uint32_t bv = (uint32_t)lo;
-            w4[j >> 2] |= bv << (8 * (j & 3));
-            if (out_fm) out_fm[(size_t)f * ld_fm + r] = (uint8_t)bv;
-            if (out_imp) out_imp[(size_t)r * ld_imp + f] = x;
+            int k[U];
+            const float* e[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (isnan(x[u])) x[u] = s_med[jj[u]];
+                if (A.imp && i0 + u * TT < total) A.imp[(size_t)(r0 + rr[u]) * A.ld_imp + f0 + jj[u]] = x[u];
+                k[u] = 1;
+                e[u] = s_e + jj[u] * TSTRIDE;
+            }
+            for (int lv = 0; lv < levels; ++lv) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) k[u] = 2 * k[u] + (e[u][k[u]] < x[u] ? 1 : 0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i0 + u * TT < total) s_b[jj[u] * TBYTES + rr[u]] = (uint8_t)(k[u] - nodes);
         }
-        if (out_rm) {
-            uint8_t* dst = out_rm + (size_t)r * ld_rm + f0;
-            if (rm_vec) {
-                *reinterpret_cast<uint4*>(dst) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
-            } else {
-                for (int j = 0; j < HT && f0 + j < F; ++j) dst[j] = (uint8_t)(w4[j >> 2] >> (8 * (j & 3)));
+        __syncthreads();
+        if (A.fm) {
+            for (int i = tid; i < nf * (TR / 16); i += TT) {
+                const int jf = i / (TR / 16), r16 = (i % (TR / 16)) * 16;
+                if (r16 >= rows) continue;
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(s_b + jf * TBYTES + r16);
+                uint8_t* dst = A.fm + (size_t)(f0 + jf) * A.ld_fm + r0 + r16;
+                if (A.fm_vec && r16 + 16 <= rows) {
+                    *reinterpret_cast<uint4*>(dst) = make_uint4(src[0], src[1], src[2], src[3]);
+                } else {
+                    for (int q = 0; q < 16 && r16 + q < rows; ++q) dst[q] = s_b[jf * TBYTES + r16 + q];
+                }
+            }
+        }
+        if (A.rm && A.rm_vec) {
+            for (int i = tid; i < nq * (TR / 4); i += TT) {
+                const int q = i % nq, r4 = (i / nq) * 4;
+                uint32_t c[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    c[t] = 4 * q + t < nf ? *reinterpret_cast<const uint32_t*>(s_b + (4 * q + t) * TBYTES + r4) : 0u;
+                // byte t of row t4's word: byte t4 of feature t's word
+                const uint32_t a0 = __builtin_amdgcn_perm(c[1], c[0], 0x05010400u), a1 = __builtin_amdgcn_perm(c[1], c[0], 0x07030602u);
+                const uint32_t b0 = __builtin_amdgcn_perm(c[3], c[2], 0x05010400u), b1 = __builtin_amdgcn_perm(c[3], c[2], 0x07030602u);
+                const uint32_t o[4] = {__builtin_amdgcn_perm(b0, a0, 0x05040100u), __builtin_amdgcn_perm(b0, a0, 0x07060302u),
+                                       __builtin_amdgcn_perm(b1, a1, 0x05040100u), __builtin_amdgcn_perm(b1, a1, 0x07060302u)};
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (r4 + t < rows)
+                        *reinterpret_cast<uint32_t*>(A.rm + (size_t)(r0 + r4 + t) * A.ld_rm + f0 + 4 * q) = o[t];
+            }
+        } else if (A.rm) {
+            int jb = tid % nf, rb = tid / nf;
+            for (int i = tid; i < total; i += TT) {
+                A.rm[(size_t)(r0 + rb) * A.ld_rm + f0 + jb] = s_b[jb * TBYTES + rb];
+                jb += dj;
+                rb += dr;
+                if (jb >= nf) {
+                    jb -= nf;
+                    ++rb;
+                }
             }
         }
     }
@@ -502,14 +602,19 @@ int yabt_bin_transform(const float* X, int64_t ldx, int64_t n, int F, const floa
     if (n < 0 || F < 1 || ldx < F || ld_edges < 1 || (out_fm && ld_fm < n) || (out_imputed && ld_imputed < F))
         return fail(-2, "yabt_bin_transform: bad sizes");
     if (out_rm && ld_rm < F) return fail(-2, "yabt_bin_transform: row-major output needs ld_rm >= F");
-    // 16-byte row stores when every 16-feature tile of every row is 16-byte aligned
-    const int rm_vec = out_rm && ld_rm % 16 == 0 && aligned16(out_rm) ? 1 : 0;
     if (!X || !edges || !nedges || !medians || !(out_fm || out_rm || out_imputed))
         return fail(-2, "yabt_bin_transform: null pointer argument");
     if (n == 0) return 0;
-    const dim3 grid((unsigned)launch_grid(n, TB, 4096), (unsigned)((F + HT - 1) / HT));
-    k_transform<<<grid, TB, 0, stream>>>(X, ldx, n, F, edges, ld_edges, nedges, medians, out_fm, ld_fm, out_rm, ld_rm,
-                                         out_imputed, ld_imputed, rm_vec);
+    const int groups = (F + TFEAT - 1) / TFEAT;
+    const int fg = ((F + groups - 1) / groups + 3) / 4 * 4;
+    // 16-byte row stores when every 16-feature tile of every row is 16-byte aligned
+    const TransformArgs A{X, ldx, n, F, fg, edges, ld_edges, nedges, medians, out_fm, ld_fm, out_rm, ld_rm, out_imputed,
+                          ld_imputed, out_fm && ld_fm % 16 == 0 && aligned16(out_fm),
+                          out_rm && ld_rm % 16 == 0 && aligned16(out_rm)};
+    const size_t lds = (size_t)fg * (TSTRIDE * 4 + 4 + TBYTES);
+    // two blocks a CU stay for all tiles: each loads its edges once
+    const dim3 grid((unsigned)launch_grid(n, TR, std::max(1, 512 / ((F + fg - 1) / fg))), (unsigned)((F + fg - 1) / fg));
+    k_transform<<<grid, TT, lds, stream>>>(A);
     return launch_status("yabt_bin_transform launch");
 }
 
