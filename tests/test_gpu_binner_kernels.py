@@ -41,3 +41,64 @@ def test_transform_equals_searchsorted(n, F, longest):
     wide = torch.zeros((n, F + 3), device=dev)                             # a column stride of 1, a longer row
     wide[:, :F] = Xd
     assert np.array_equal(b.transform(wide[:, :F]).cpu().numpy(), want)
+
+
+def _column(rng, kind, n):
+    if kind == "normal":
+        x = rng.normal(size=n)
+    elif kind == "counts":           # ties of every size, one of them the median's
+        x = np.floor(rng.exponential(3.0, size=n))
+    elif kind == "zeros":            # zero IQR: the std fallback
+        x = np.where(rng.random(n) < 0.9, 0.0, rng.normal(size=n))
+    elif kind == "half":             # the median's two values lie in two far blocks of ties
+        x = np.where(np.arange(n) % 2 == 0, -1.0, 3.0)
+    elif kind == "narrow":           # keys that differ in their last bits only
+        x = 1.0 + rng.integers(0, 50, size=n) * 2.0 ** -23
+    else:                            # "constant"
+        x = np.full(n, 2.5)
+    return x.astype(np.float32)
+
+
+KINDS = ["normal", "counts", "zeros", "half", "narrow", "constant"]
+
+
+@pytest.mark.parametrize("n,missing", [(2, 0.0), (4095, 0.0), (4096, 0.3), (4097, 0.0), (8193, 0.01), (65537, 0.5),
+                                       (200_001, 0.0), (200_002, 0.2), (900_001, 0.05)])
+def test_fit_equals_numpy(n, missing):
+    """Sort chunks' edges, the std fallback's buffers (whole, partial, with NaN
+    gaps) and the medians' brackets, against the oracle's numpy binner."""
+    from oracle import boost_oracle as BO
+    rng = np.random.default_rng(n)
+    X = np.stack([_column(rng, k, n) for k in KINDS], axis=1)
+    X[rng.random(X.shape) < missing] = np.nan
+    ref, b = BO.Binner(256).fit(X), Binner(256).fit(X)
+    for f in range(X.shape[1]):
+        want = ref.edges_[f].astype(np.float32)
+        assert np.array_equal(b.edges_[f].numpy().view(np.uint32), want.view(np.uint32)), KINDS[f]
+    assert np.array_equal(b.scales_.numpy().view(np.uint32), ref.scales_.view(np.uint32))
+    assert np.array_equal(b.medians_.view(np.uint32), np.nanmedian(X, axis=0).astype(np.float32).view(np.uint32))
+
+
+def test_medians_of_a_sample_that_is_not_random():
+    """The C entry takes any rows as the sample: the medians are of all rows."""
+    import ctypes
+    from yabt_amd import _lib
+    rng = np.random.default_rng(5)
+    n, F, m = 30_000, 300, 5000
+    X = rng.normal(size=(n, F)).astype(np.float32)
+    X = np.sort(X, axis=0)
+    X[:, 7] = np.nan
+    dev = torch.device("cuda", 0)
+    Xd, rows = torch.from_numpy(X).to(dev), torch.arange(m, device=dev)     # the smallest values
+    lib = _lib.load()
+    nb = int(lib.yabt_bin_fit_workspace_bytes(m, F))
+    ws = torch.empty(nb, dtype=torch.uint8, device=dev)
+    edges, ne = torch.empty((F, 255), device=dev), torch.empty(F, dtype=torch.int32, device=dev)
+    sc, med = torch.empty(F, device=dev), torch.empty(F, device=dev)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    _lib.check(lib.yabt_bin_fit(p(Xd), F, n, F, p(rows), m, 256, p(ws), nb, p(edges), 255, p(ne), p(sc), p(med),
+                                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "yabt_bin_fit")
+    want = np.zeros(F, np.float32)
+    keep = np.arange(F) != 7
+    want[keep] = np.median(X[:, keep], axis=0)
+    assert np.array_equal(med.cpu().numpy().view(np.uint32), want.view(np.uint32))

@@ -10,13 +10,14 @@
 //                       layouts, plus the imputed fp32 matrix
 //
 // Fit, per feature: the sample column is gathered as order-preserving uint32
-// keys (NaN last), sorted by a stable 4 x 8-bit radix sort (one block per
-// feature), and the quantiles are read off the sorted keys with numpy's
-// arithmetic: virtual index (c - 1) * q in double, d = fp32(b - a), value
+// keys (NaN last), sorted by a stable 4 x 8-bit radix sort, and the quantiles
+// are read off the sorted keys with numpy's arithmetic: virtual index (c - 1) * q in double, d = fp32(b - a), value
 // a + d * t (t < 1/2) or b - d * (1 - t) in double (numpy _lerp), rounded to
 // fp32; the edges are those values sorted and de-duplicated (np.unique).
-// Medians: a 4-pass radix select of the two middle order statistics over all
-// rows, combined as numpy's float32 mean of two values.
+// Medians: of all rows, from the sorted keys when the sample is all rows, else
+// from one pass over X that counts around a bracket taken from the sample and
+// keeps what lies inside it; a 4-pass radix select over all rows when a
+// bracket missed.  The two middle values are combined as numpy's float32 mean.
 
 #include "common.h"
 #include "host.h"
@@ -29,13 +30,16 @@
 namespace yabt {
 namespace bin {
 
-constexpr int SB = 1024;            // sort block
+constexpr int RT = 256;             // threads of a sort block
+constexpr int RK = 16;              // keys per thread
+constexpr int RC = RT * RK;         // keys per sort block
 constexpr int HT = 16;              // features per histogram tile
 constexpr int TB = 256;             // threads per select block
 constexpr int MAXE = 255;           // edges per feature (max_bins - 1 <= 255)
+constexpr uint32_t NAN_KEY = 0xFFFFFFFFu;
 
 __device__ __forceinline__ uint32_t fkey(float v) {
-    if (isnan(v)) return 0xFFFFFFFFu;
+    if (isnan(v)) return NAN_KEY;
     const uint32_t b = __float_as_uint(v);
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
@@ -44,13 +48,28 @@ __device__ __forceinline__ float kval(uint32_t k) {
     return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
 
+// Bracket of a feature's median and what the pass over all rows finds about it.
+struct Bracket {
+    uint32_t lo, hi;       // keys; lo == hi: one value
+    uint32_t below;        // rows with key < lo
+    uint32_t eq_lo, eq_hi; // rows with key lo, and key hi (> lo)
+    uint32_t inside;       // rows between: list entries wanted (may exceed the list)
+    uint32_t valid;        // non-NaN rows
+    uint32_t pad;
+};
+
 struct FitWs {
     uint32_t* orig;        // (F, m) sample keys in sample order
     uint32_t* ka;          // (F, m) sorted keys
-    uint32_t* kb;          // (F, m) radix ping-pong, then the std fallback's scratch
+    uint32_t* kb;          // (F, m) radix ping-pong, then the std fallback's column, then the median lists
+    uint32_t* dig;         // (F, 256, chunks) digit counts, then places
+    uint32_t* need_std;    // (F) the IQR was 0
+    Bracket* br;           // (F)
     uint32_t* cnt;         // (F) non-NaN rows over all n
+    uint32_t* missed;      // (1) some bracket missed: select over all rows
     uint32_t* sel_hist;    // (F, 2, 256)
     uint32_t* sel_state;   // (F, 2, 2): prefix, rank
+    int64_t chunks;
     size_t bytes;
 };
 
@@ -58,148 +77,197 @@ FitWs carve_fit(char* base, int64_t m, int F) {
     Carve c{base, 0};
     FitWs w;
     const size_t fm = (size_t)F * (size_t)(m > 0 ? m : 1);
+    w.chunks = (m + RC - 1) / RC;
     w.orig = c.take<uint32_t>(fm);
     w.ka = c.take<uint32_t>(fm);
     w.kb = c.take<uint32_t>(fm);
+    w.dig = c.take<uint32_t>(w.chunks > 1 ? (size_t)F * NB * (size_t)w.chunks : 1);
+    w.need_std = c.take<uint32_t>(F);
+    w.br = c.take<Bracket>(F);
     w.cnt = c.take<uint32_t>(F);
+    w.missed = c.take<uint32_t>(1);
     w.sel_hist = c.take<uint32_t>((size_t)F * 2 * NB);
     w.sel_state = c.take<uint32_t>((size_t)F * 4);
     w.bytes = c.off;
     return w;
 }
 
-// keys[f][i] = key of X[rows[i]][f] (rows == null: row i).
+// keys[f][i] = key of X[rows[i]][f] (rows == null: row i): 64 rows x 64
+// features turned in LDS, so that rows are read and columns written in runs.
 __global__ void __launch_bounds__(TB) k_gather_keys(const float* __restrict__ X, int64_t ldx, int F,
                                                     const int64_t* __restrict__ rows, int64_t m,
                                                     uint32_t* __restrict__ keys) {
-    const int64_t total = m * F;
-    for (int64_t t = (int64_t)blockIdx.x * TB + threadIdx.x; t < total; t += (int64_t)gridDim.x * TB) {
-        const int64_t i = t / F;
-        const int f = (int)(t - i * F);
-        const int64_t r = rows ? rows[i] : i;
-        keys[(size_t)f * m + i] = fkey(X[(size_t)r * ldx + f]);
+    __shared__ uint32_t s_k[64][65];
+    const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
+    const int64_t i0 = (int64_t)blockIdx.x * 64;
+    const int f0 = blockIdx.y * 64;
+    if (f0 + lane < F) {
+#pragma unroll 8
+        for (int q = 0; q < 16; ++q) {
+            const int64_t i = min(i0 + w * 16 + q, m - 1);
+            const int64_t r = rows ? rows[i] : i;
+            s_k[lane][w * 16 + q] = fkey(X[(size_t)r * ldx + f0 + lane]);
+        }
     }
+    __syncthreads();
+    if (i0 + lane < m)
+        for (int j = w; j < 64 && f0 + j < F; j += TB / 64) keys[(size_t)(f0 + j) * m + i0 + lane] = s_k[j][lane];
 }
 
-// Stable LSD radix sort of each feature's m keys, one block per feature.
-// Result in a (4 passes: a -> b -> a -> b -> a).
-__global__ void __launch_bounds__(SB) k_sort(uint32_t* __restrict__ ka, uint32_t* __restrict__ kb, int64_t m) {
-    __shared__ uint32_t s_base[NB];
-    __shared__ uint32_t s_tot[NB];
-    __shared__ uint32_t s_wc[SB / WAVE][NB];
-    const int f = blockIdx.x, tid = threadIdx.x, w = tid / WAVE;
-    uint32_t* a = ka + (size_t)f * m;
-    uint32_t* b = kb + (size_t)f * m;
-    for (int pass = 0; pass < 4; ++pass) {
-        const int shift = 8 * pass;
-        const uint32_t* src = (pass & 1) ? b : a;
-        uint32_t* dst = (pass & 1) ? a : b;
-        if (tid < NB) s_tot[tid] = 0;
-        __syncthreads();
-        for (int64_t i = tid; i < m; i += SB) atomicAdd(&s_tot[(src[i] >> shift) & 255u], 1u);
-        __syncthreads();
-        if (tid == 0) {                  // digit starts: exclusive prefix of the counts
-            uint32_t run = 0;
-            for (int d = 0; d < NB; ++d) {
-                const uint32_t c = s_tot[d];
-                s_base[d] = run;
-                run += c;
-            }
-        }
-        __syncthreads();
-        for (int64_t t0 = 0; t0 < m; t0 += SB) {
-            for (int j = tid; j < (SB / WAVE) * NB; j += SB) (&s_wc[0][0])[j] = 0;
-            __syncthreads();
-            const int64_t i = t0 + tid;
-            const bool v = i < m;
-            const uint32_t key = v ? src[i] : 0u;
-            const uint32_t d = (key >> shift) & 255u;
-            uint64_t peers = __ballot(v);
+// ---------------------------------------------------------------------------
+// stable LSD radix sort of each feature's m keys, 4 passes of 8 bits.  A block
+// takes RC keys: wave w's keys are RK rounds of 64 neighbours, so a key's rank
+// among the block's equal digits is the wave's running count of the digit plus
+// the lanes before it (eight ballots), with no barrier until the wave's keys
+// are done.  One block sorts up to RC keys in LDS; above that a pass is a
+// count, a scan of (digit, chunk) and a scatter through LDS that writes each
+// digit's keys in a run.  200 000 x 50: 1607 us by one block per feature,
+// which walked its tiles one after the other with five barriers each (50 of
+// 256 CUs busy), 272 us by chunks
+// (scatters 145, counts 90, scans 37).
+// ---------------------------------------------------------------------------
+
+struct RadixLds {
+    uint32_t wc[RT / WAVE][NB];    // running counts, then the wave's start among the block's equal digits
+    uint32_t start[NB];            // the digit's first place in the block
+    uint32_t keys[RC];
+    uint32_t scan[RT / WAVE];
+};
+
+// Places of the block's keys sorted by digit; keys past the end are NAN_KEY
+// (the highest digit, after all others).
+__device__ __forceinline__ void radix_places(RadixLds& L, const uint32_t (&key)[RK], int shift, uint32_t (&place)[RK]) {
+    const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+    for (int i = threadIdx.x; i < (RT / WAVE) * NB; i += RT) (&L.wc[0][0])[i] = 0;
+    __syncthreads();
+    volatile uint32_t* wc = L.wc[w];
 #pragma unroll
-            for (int bit = 0; bit < 8; ++bit) {
-                const bool on = (d >> bit) & 1u;
-                const uint64_t bal = __ballot(on);
-                peers &= on ? bal : ~bal;
-            }
-            const uint32_t rk = lane_prefix(peers);
-            if (v && rk == 0) s_wc[w][d] = (uint32_t)__popcll(peers);
-            __syncthreads();
-            if (tid < NB) {
-                uint32_t run = 0;
-                for (int k = 0; k < SB / WAVE; ++k) {
-                    const uint32_t c = s_wc[k][tid];
-                    s_wc[k][tid] = run;
-                    run += c;
-                }
-                s_tot[tid] = run;
-            }
-            __syncthreads();
-            if (v) dst[s_base[d] + s_wc[w][d] + rk] = key;
-            __syncthreads();
-            if (tid < NB) s_base[tid] += s_tot[tid];
-            __syncthreads();
+    for (int q = 0; q < RK; ++q) {
+        const uint32_t d = (key[q] >> shift) & 255u;
+        uint64_t peers = ~0ull;
+#pragma unroll
+        for (int bit = 0; bit < 8; ++bit) {
+            const bool on = (d >> bit) & 1u;
+            const uint64_t bal = __ballot(on);
+            peers &= on ? bal : ~bal;
         }
+        const uint32_t before = lane_prefix(peers), run = wc[d];
+        place[q] = run + before;
+        __builtin_amdgcn_wave_barrier();       // every lane has read its count
+        if (before == 0) wc[d] = run + (uint32_t)__popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    uint32_t run = 0;
+#pragma unroll
+    for (int k = 0; k < RT / WAVE; ++k) {      // thread d: digit d
+        const uint32_t c = L.wc[k][threadIdx.x];
+        L.wc[k][threadIdx.x] = run;
+        run += c;
+    }
+    uint32_t tot;
+    L.start[threadIdx.x] = block_excl_scan<RT, uint32_t>(run, L.scan, &tot);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RK; ++q) {
+        const uint32_t d = (key[q] >> shift) & 255u;
+        place[q] += L.start[d] + L.wc[w][d];
+    }
+    (void)lane;
+}
+
+__device__ __forceinline__ int64_t radix_index(int q) {
+    return (int64_t)(threadIdx.x / WAVE) * (RC / (RT / WAVE)) + q * WAVE + threadIdx.x % WAVE;
+}
+
+// m <= RC: the whole sort in one block per feature.
+__global__ void __launch_bounds__(RT) k_sort_small(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst,
+                                                   int64_t m) {
+    __shared__ RadixLds L;
+    src += (size_t)blockIdx.x * m;
+    dst += (size_t)blockIdx.x * m;
+    uint32_t key[RK], place[RK];
+#pragma unroll
+    for (int q = 0; q < RK; ++q) key[q] = radix_index(q) < m ? src[radix_index(q)] : NAN_KEY;
+    for (int shift = 0; shift < 32; shift += 8) {
+        radix_places(L, key, shift, place);
+#pragma unroll
+        for (int q = 0; q < RK; ++q) L.keys[place[q]] = key[q];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < RK; ++q) key[q] = L.keys[radix_index(q)];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < RK; ++q)
+        if (radix_index(q) < m) dst[radix_index(q)] = key[q];
+}
+
+// dig[f][digit][chunk] = the chunk's keys with that digit.
+__global__ void __launch_bounds__(RT) k_radix_count(const uint32_t* __restrict__ src, int64_t m, int shift,
+                                                    int64_t chunks, uint32_t* __restrict__ dig) {
+    __shared__ uint32_t s_c[NB];
+    const int64_t chunk = blockIdx.x % chunks, f = blockIdx.x / chunks, c0 = chunk * RC;
+    src += (size_t)f * m;
+    s_c[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RK; ++q) {
+        const int64_t i = c0 + q * RT + threadIdx.x;
+        if (i < m) atomicAdd(&s_c[(src[i] >> shift) & 255u], 1u);
+    }
+    __syncthreads();
+    dig[((size_t)f * NB + threadIdx.x) * chunks + chunk] = s_c[threadIdx.x];
+}
+
+// Exclusive prefix of a feature's (digit, chunk) counts.
+__global__ void __launch_bounds__(1024) k_radix_scan(uint32_t* __restrict__ dig, int64_t chunks) {
+    __shared__ uint32_t s_w[1024 / WAVE];
+    uint32_t* d = dig + (size_t)blockIdx.x * NB * chunks;
+    const int64_t total = NB * chunks;
+    uint32_t carry = 0;
+    for (int64_t base = 0; base < total; base += 1024 * 4) {
+        const int64_t i = base + threadIdx.x * 4;
+        uint32_t v[4], sum = 0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            v[t] = i + t < total ? d[i + t] : 0u;
+            sum += v[t];
+        }
+        uint32_t tot;
+        uint32_t run = carry + block_excl_scan<1024, uint32_t>(sum, s_w, &tot);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            if (i + t < total) d[i + t] = run;
+            run += v[t];
+        }
+        carry += tot;
     }
 }
 
-// numpy's float32 pairwise sum of one buffer, iteratively: blocks of <= 128
-// summed with eight accumulators, halves split at multiples of 8.
-__device__ float np_pairwise_sum(const float* a, int64_t n) {
-    struct Fr {
-        int64_t off, n;
-        int stage;
-        float left;
-    };
-    Fr st[40];
-    int sp = 0;
-    st[0] = Fr{0, n, 0, 0.0f};
-    float ret = 0.0f;
-    while (true) {
-        Fr& fr = st[sp];
-        if (fr.stage == 0 && fr.n > 128) {
-            int64_t n2 = fr.n / 2;
-            n2 -= n2 % 8;
-            fr.stage = 1;
-            st[sp + 1] = Fr{fr.off, n2, 0, 0.0f};
-            ++sp;
-            continue;
-        }
-        if (fr.stage == 1) {               // left half done: ret holds it
-            fr.left = ret;
-            fr.stage = 2;
-            int64_t n2 = fr.n / 2;
-            n2 -= n2 % 8;
-            st[sp + 1] = Fr{fr.off + n2, fr.n - n2, 0, 0.0f};
-            ++sp;
-            continue;
-        }
-        float res;
-        if (fr.stage == 2) {
-            res = fr.left + ret;
-        } else if (fr.n < 8) {
-            res = 0.0f;
-            for (int64_t i = 0; i < fr.n; ++i) res += a[fr.off + i];
-        } else {
-            float r[8];
-            for (int j = 0; j < 8; ++j) r[j] = a[fr.off + j];
-            int64_t i = 8;
-            for (; i < fr.n - (fr.n % 8); i += 8)
-                for (int j = 0; j < 8; ++j) r[j] += a[fr.off + i + j];
-            res = ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]));
-            for (; i < fr.n; ++i) res += a[fr.off + i];
-        }
-        ret = res;
-        if (sp == 0) return ret;
-        --sp;
+__global__ void __launch_bounds__(RT) k_radix_scatter(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst,
+                                                      int64_t m, int shift, int64_t chunks,
+                                                      const uint32_t* __restrict__ dig) {
+    __shared__ RadixLds L;
+    __shared__ uint32_t s_to[NB];              // the digit's first place in dst, less its place in the block
+    const int64_t chunk = blockIdx.x % chunks, f = blockIdx.x / chunks, c0 = chunk * RC;
+    src += (size_t)f * m;
+    dst += (size_t)f * m;
+    const uint32_t to = dig[((size_t)f * NB + threadIdx.x) * chunks + chunk];
+    uint32_t key[RK], place[RK];
+#pragma unroll
+    for (int q = 0; q < RK; ++q) key[q] = c0 + radix_index(q) < m ? src[c0 + radix_index(q)] : NAN_KEY;
+    radix_places(L, key, shift, place);
+    s_to[threadIdx.x] = to - L.start[threadIdx.x];
+#pragma unroll
+    for (int q = 0; q < RK; ++q) L.keys[place[q]] = key[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RK; ++q) {
+        const uint32_t i = q * RT + threadIdx.x, k = L.keys[i];
+        const uint32_t at = s_to[(k >> shift) & 255u] + i;
+        if (at < (uint32_t)m) dst[at] = k;     // past the end: the filled-up keys
     }
-}
-
-// numpy's float32 sum of a contiguous array: 8192-element buffers, each
-// summed pairwise, added in order to an accumulator that starts at 0.
-__device__ float np_sum(const float* a, int64_t n) {
-    float acc = 0.0f;
-    for (int64_t i = 0; i < n; i += 8192) acc += np_pairwise_sum(a + i, min((int64_t)8192, n - i));
-    return acc;
 }
 
 // numpy's linear quantile of the c sorted keys at q (numpy _quantile/_lerp),
@@ -222,39 +290,55 @@ __device__ double np_quantile(const uint32_t* sk, int64_t c, double q) {
     return t >= 0.5 ? (double)b - (double)d * (1.0 - t) : (double)a + (double)d * t;
 }
 
-// One block per feature: edges, edge count, scale.
-__global__ void __launch_bounds__(TB) k_quantiles(const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ orig,
-                                                  float* __restrict__ scratch, int64_t m, int max_bins,
+// One block per feature: edges, edge count, scale (or the wish for the std
+// fallback); the median when the sample is all rows, else its bracket.
+__global__ void __launch_bounds__(TB) k_quantiles(const uint32_t* __restrict__ sorted, int64_t m, int max_bins, int whole,
                                                   float* __restrict__ out_edges, int64_t ld_edges,
-                                                  int32_t* __restrict__ out_nedges, float* __restrict__ out_scales) {
-    __shared__ float s_q[MAXE];
-    __shared__ uint32_t s_c;
+                                                  int32_t* __restrict__ out_nedges, float* __restrict__ out_scales,
+                                                  float* __restrict__ out_medians, uint32_t* __restrict__ need_std,
+                                                  Bracket* __restrict__ br, uint32_t* __restrict__ missed) {
+    __shared__ float s_q[TB];
+    __shared__ int s_wave[TB / WAVE];
+    __shared__ int64_t s_lo, s_hi;
+    __shared__ int s_bad;
     const int f = blockIdx.x, tid = threadIdx.x;
     const uint32_t* sk = sorted + (size_t)f * m;
-    if (tid == 0) {                         // non-NaN keys sort below 0xFFFFFFFF
-        int64_t lo = 0, hi = m;
-        while (lo < hi) {
-            const int64_t mid = (lo + hi) / 2;
-            if (sk[mid] != 0xFFFFFFFFu) lo = mid + 1;
-            else hi = mid;
-        }
-        s_c = (uint32_t)lo;
+    if (tid == 0) {
+        s_lo = 0;                           // non-NaN keys sort below NAN_KEY: their count lies in [lo, hi]
+        s_hi = m;
+        s_bad = 0;
     }
     __syncthreads();
-    const int64_t c = s_c;
+    while (s_hi > s_lo) {                   // TB probes a round
+        const int64_t lo = s_lo, hi = s_hi, step = (hi - lo + TB - 1) / TB, at = lo + tid * step;
+        const bool num = at < hi && sk[at] != NAN_KEY;
+        const int n = block_sum<TB, int>(num ? 1 : 0, s_wave);   // the first n probes are numbers
+        if (tid == 0) {
+            s_lo = n ? lo + (n - 1) * step + 1 : lo;
+            s_hi = n ? min(hi, lo + n * step) : lo;
+        }
+        __syncthreads();
+    }
+    const int64_t c = s_lo;
     const uint32_t zero_key = 0x80000000u;  // an all-NaN (or empty) column is [0.0] (binning.py:57-59)
     const uint32_t* keys = c > 0 ? sk : &zero_key;
     const int64_t cc = c > 0 ? c : 1;
     const int ne = max_bins - 1;
     const double step = 1.0 / (double)max_bins;   // np.linspace(0, 1, max_bins + 1)
-    for (int j = tid; j < ne; j += TB) {
-        const double q = (double)(j + 1) * step + 0.0;
-        s_q[j] = (float)np_quantile(keys, cc, q);
+    if (tid < ne) {
+        const double q = (double)(tid + 1) * step + 0.0;
+        s_q[tid] = (float)np_quantile(keys, cc, q);
     }
     __syncthreads();
-    if (tid == 0) {
-        // np.unique: sort (insertion; the values are already nearly sorted;
-        // NaN last) and drop repeats (NaNs count as equal)
+    // np.unique: sort (NaN last) and drop repeats (NaNs count as equal).  The
+    // values come in order but for the rounding of neighbours; only then one
+    // thread sorts them.
+    if (tid + 1 < ne) {
+        const float v = s_q[tid + 1], p = s_q[tid];
+        if (isnan(v) ? false : (isnan(p) || p > v)) s_bad = 1;
+    }
+    __syncthreads();
+    if (s_bad && tid == 0) {
         for (int i = 1; i < ne; ++i) {
             const float v = s_q[i];
             int k = i - 1;
@@ -264,60 +348,335 @@ __global__ void __launch_bounds__(TB) k_quantiles(const uint32_t* __restrict__ s
             }
             s_q[k + 1] = v;
         }
-        int u = 0;
-        for (int i = 0; i < ne; ++i)
-            if (i == 0 || !(s_q[i] == s_q[u - 1] || (isnan(s_q[i]) && isnan(s_q[u - 1])))) s_q[u++] = s_q[i];
+    }
+    __syncthreads();
+    const float v = tid < ne ? s_q[tid] : 0.0f;
+    int keep = 0;
+    if (tid < ne) keep = tid == 0 || !(v == s_q[tid - 1] || (isnan(v) && isnan(s_q[tid - 1])));
+    int u;
+    const int at = block_excl_scan<TB, int>(keep, s_wave, &u);
+    if (keep) out_edges[(size_t)f * ld_edges + at] = v;
+    if (tid == 0) {
         out_nedges[f] = u;
-        for (int i = 0; i < u; ++i) out_edges[(size_t)f * ld_edges + i] = s_q[i];
         // scale: q75 - q25 in double, else numpy's float32 std of the column, else 1
-        double s = np_quantile(keys, cc, 0.75) - np_quantile(keys, cc, 0.25);
-        if (s == 0.0) {
-            float* col = scratch + (size_t)f * m;
-            int64_t k = 0;
-            const uint32_t* ok = orig + (size_t)f * m;
-            for (int64_t i = 0; i < m; ++i)
-                if (ok[i] != 0xFFFFFFFFu) col[k++] = kval(ok[i]);
-            if (k == 0) col[k++] = 0.0f;
-            const float mean = np_sum(col, k) / (float)k;
-            for (int64_t i = 0; i < k; ++i) {
-                const float x = col[i] - mean;
-                col[i] = x * x;
-            }
-            const float var = np_sum(col, k) / (float)k;
-            s = (double)sqrtf(var);
-            if (s == 0.0) s = 1.0;
-        }
+        const double s = np_quantile(keys, cc, 0.75) - np_quantile(keys, cc, 0.25);
+        need_std[f] = s == 0.0;
         out_scales[f] = (float)s;
+    }
+    if (tid == 1) {
+        if (whole) {
+            // np.nanmedian of the rows, 0 where all are NaN (binning.py:32-33)
+            float med = 0.0f;
+            if (c > 0) {
+                const float a = kval(sk[(c - 1) / 2]), b = kval(sk[c / 2]);
+                med = (c % 2) ? a : (a + b) / 2.0f;
+                if (isnan(med)) med = 0.0f;
+            }
+            out_medians[f] = med;
+        } else {
+            // the rows' median lies within 3 sqrt(c) sample ranks of the
+            // sample's (six standard deviations of a random sample's)
+            Bracket b = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+            if (c > 0) {
+                const int64_t mid = (c - 1) / 2, w = (int64_t)(3.0 * sqrt((double)c)) + 8;
+                b.lo = mid >= w ? sk[mid - w] : 0u;
+                b.hi = mid + 1 + w < c ? sk[mid + 1 + w] : NAN_KEY - 1;
+            }
+            br[f] = b;
+        }
+    }
+    if (f == 0 && tid == 2) *missed = 0;
+}
+
+// ---------------------------------------------------------------------------
+// scale of a column whose IQR is zero: numpy's float32 std, in its order --
+// 8192-element buffers, each summed pairwise (halves split at multiples of 8
+// down to at most 128 elements, those with eight accumulators), added in order
+// to an accumulator that starts at 0.  A buffer's at most 128 runs are summed
+// by 128 threads and combined along the same splits.
+// ---------------------------------------------------------------------------
+constexpr int PB = 8192;                    // elements per buffer
+constexpr int PL = 128;                     // elements per run; also the most runs of a buffer
+constexpr int PD = 7;                       // levels of splits
+constexpr int ST = 1024;                    // threads: eight buffers at a time
+
+// The run that path (PD bits, first split highest) leads to in a buffer of n
+// elements: its place and length; false when it is another path's (a run that
+// ends above the last split is its all-zero path's).  level: stop there.
+__device__ __forceinline__ bool pairwise_run(int path, int level, int n, int* off, int* len) {
+    int o = 0;
+    for (int d = 0; d < level; ++d) {
+        const int bit = (path >> (PD - 1 - d)) & 1;
+        if (n <= PL) {
+            if (bit) return false;
+            continue;
+        }
+        int h = n / 2;
+        h -= h % 8;
+        o += bit ? h : 0;
+        n = bit ? n - h : h;
+    }
+    *off = o;
+    *len = n;
+    return true;
+}
+
+template <typename Get>
+__device__ float pairwise_leaf(const Get& get, int64_t off, int n) {
+    if (n < 8) {
+        float res = 0.0f;
+        for (int i = 0; i < n; ++i) res += get(off + i);
+        return res;
+    }
+    float r[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) r[j] = get(off + j);
+    int i = 8;
+    for (; i < n - (n % 8); i += 8)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) r[j] += get(off + i + j);
+    float res = ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]));
+    for (; i < n; ++i) res += get(off + i);
+    return res;
+}
+
+// numpy's float32 sum of get(0 .. k - 1), by the block.
+template <typename Get>
+__device__ float block_np_sum(const Get& get, int64_t k, float (*s_v)[PL]) {
+    const int buf = threadIdx.x / PL, path = threadIdx.x % PL;
+    float acc = 0.0f;
+    for (int64_t b0 = 0; b0 < k; b0 += (int64_t)PB * (ST / PL)) {
+        const int64_t first = b0 + (int64_t)buf * PB;
+        const int n = (int)max((int64_t)0, min((int64_t)PB, k - first));
+        int off, len;
+        if (n > 0 && pairwise_run(path, PD, n, &off, &len)) s_v[buf][path] = pairwise_leaf(get, first + off, len);
+        __syncthreads();
+        for (int d = PD - 1; d >= 0; --d) {    // the splits of level d
+            const int half = 1 << (PD - 1 - d);
+            if (n > 0 && path % (2 * half) == 0 && pairwise_run(path, d, n, &off, &len) && len > PL)
+                s_v[buf][path] = s_v[buf][path] + s_v[buf][path + half];
+            __syncthreads();
+        }
+        for (int j = 0; j < ST / PL && b0 + (int64_t)j * PB < k; ++j) acc += s_v[j][0];
+        __syncthreads();
+    }
+    return acc;
+}
+
+__global__ void __launch_bounds__(ST) k_std_scale(const uint32_t* __restrict__ orig, float* __restrict__ scratch, int64_t m,
+                                                  const uint32_t* __restrict__ need_std, float* __restrict__ out_scales) {
+    __shared__ float s_v[ST / PL][PL];
+    __shared__ uint32_t s_wave[ST / WAVE];
+    const int f = blockIdx.x, tid = threadIdx.x;
+    if (!need_std[f]) return;
+    const uint32_t* ok = orig + (size_t)f * m;
+    float* col = scratch + (size_t)f * m;
+    int64_t k = 0;                             // the column's numbers, in sample order
+    for (int64_t i0 = 0; i0 < m; i0 += ST * 4) {
+        uint32_t key[4], n = 0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int64_t i = i0 + tid * 4 + t;
+            key[t] = i < m ? ok[i] : NAN_KEY;
+            n += key[t] != NAN_KEY;
+        }
+        uint32_t tot;
+        int64_t at = k + block_excl_scan<ST, uint32_t>(n, s_wave, &tot);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (key[t] != NAN_KEY) col[at++] = kval(key[t]);
+        k += tot;
+    }
+    if (k == 0) {                              // an all-NaN column is [0.0]: std 0
+        if (tid == 0) out_scales[f] = 1.0f;
+        return;
+    }
+    __syncthreads();
+    const float mean = block_np_sum([&](int64_t i) { return col[i]; }, k, s_v) / (float)k;
+    const float var = block_np_sum([&](int64_t i) { const float x = col[i] - mean; return x * x; }, k, s_v) / (float)k;
+    if (tid == 0) {
+        const float s = sqrtf(var);
+        out_scales[f] = (double)s == 0.0 ? 1.0f : s;
     }
 }
 
 // ---------------------------------------------------------------------------
-// medians over all rows: radix select of the two middle order statistics
+// medians over all rows by the sample's bracket
 // ---------------------------------------------------------------------------
 
-// Non-NaN count per feature.
-__global__ void __launch_bounds__(TB) k_count_valid(const float* __restrict__ X, int64_t ldx, int64_t n, int F,
-                                                    uint32_t* __restrict__ cnt) {
-    __shared__ uint32_t s_c[HT];
-    const int f0 = blockIdx.y * HT;
-    if (threadIdx.x < HT) s_c[threadIdx.x] = 0;
+// One pass over X, every thread one feature (neighbouring threads neighbouring
+// features): rows below, at and between the bracket's ends; the keys between
+// go into the feature's list (cap places).  About 6 sqrt(c) / c of the rows lie
+// between (1.3% at a sample of 200 000), whatever ties there are: a value that
+// holds more of them than that is an end of the bracket.  2M x 50: 215 us (1.9
+// TB/s of X) and 23 us for the lists' selects; counting the numbers and
+// four digit passes over X took 1580 us and 170 us of steps between them.
+constexpr int MT = 256;                        // threads
+constexpr int MPEND = 12;                      // keys a thread holds back
+__global__ void __launch_bounds__(MT) k_median_pass(const float* __restrict__ X, int64_t ldx, int64_t n, int F, int fw,
+                                                    Bracket* __restrict__ br, uint32_t* __restrict__ lists, int64_t cap) {
+    __shared__ uint32_t s_pend[MPEND][MT];
+    __shared__ uint32_t s_c[5][MT];            // below, eq_lo, eq_hi, valid, pending of a feature
+    __shared__ uint32_t s_base[MT];
+    const int tid = threadIdx.x, j = tid % fw, f = blockIdx.y * fw + j;
+    const int per = MT / fw;                   // rows a step
+    const bool live = f < F && tid < per * fw;
+    for (int k = 0; k < 5; ++k) s_c[k][tid] = 0;
     __syncthreads();
-    const int j = threadIdx.x % HT;
-    const int f = f0 + j;
-    uint32_t c = 0;
-    if (f < F)
-        for (int64_t r = (int64_t)blockIdx.x * (TB / HT) + threadIdx.x / HT; r < n; r += (int64_t)gridDim.x * (TB / HT))
-            c += isnan(X[(size_t)r * ldx + f]) ? 0u : 1u;
-    atomicAdd(&s_c[j], c);
+    const uint32_t lo = live ? br[f].lo : 0u, hi = live ? br[f].hi : 0u;
+    uint32_t below = 0, eql = 0, eqh = 0, valid = 0, pend = 0;
+    if (live) {
+        constexpr int U = 8;
+        const int64_t step = (int64_t)gridDim.x * per;
+        for (int64_t r0 = (int64_t)blockIdx.x * per + tid / fw; r0 < n; r0 += step * U) {
+            float x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u] = r0 + u * step < n ? X[(size_t)(r0 + u * step) * ldx + f] : NAN;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t k = fkey(x[u]);
+                valid += k != NAN_KEY;
+                below += k < lo;
+                eql += k == lo;
+                eqh += k == hi && hi != lo;
+                if (k > lo && k < hi) {
+                    if (pend < MPEND) {
+                        s_pend[pend++][tid] = k;
+                    } else {
+                        const uint32_t at = atomicAdd(&br[f].inside, 1u);
+                        if (at < cap) lists[(size_t)f * cap + at] = k;
+                    }
+                }
+            }
+        }
+    }
+    uint32_t place = 0;
+    if (live) {
+        if (below) atomicAdd(&s_c[0][j], below);
+        if (eql) atomicAdd(&s_c[1][j], eql);
+        if (eqh) atomicAdd(&s_c[2][j], eqh);
+        if (valid) atomicAdd(&s_c[3][j], valid);
+        place = pend ? atomicAdd(&s_c[4][j], pend) : 0u;
+    }
     __syncthreads();
-    if (threadIdx.x < HT && f0 + threadIdx.x < F && s_c[threadIdx.x]) atomicAdd(&cnt[f0 + threadIdx.x], s_c[threadIdx.x]);
+    if (tid < fw && blockIdx.y * fw + tid < F) {
+        Bracket* b = br + blockIdx.y * fw + tid;
+        if (s_c[0][tid]) atomicAdd(&b->below, s_c[0][tid]);
+        if (s_c[1][tid]) atomicAdd(&b->eq_lo, s_c[1][tid]);
+        if (s_c[2][tid]) atomicAdd(&b->eq_hi, s_c[2][tid]);
+        if (s_c[3][tid]) atomicAdd(&b->valid, s_c[3][tid]);
+        s_base[tid] = s_c[4][tid] ? atomicAdd(&b->inside, s_c[4][tid]) : 0u;
+    }
+    __syncthreads();
+    for (uint32_t q = 0; q < pend; ++q) {
+        const uint32_t at = s_base[j] + place + q;
+        if (at < cap) lists[(size_t)f * cap + at] = s_pend[q][tid];
+    }
 }
 
+// One block per feature: the two middle order statistics from the counts and
+// the list (a radix select of the list's keys), or *missed.
+__global__ void __launch_bounds__(1024) k_median_finish(const Bracket* __restrict__ br, const uint32_t* __restrict__ lists,
+                                                        int64_t cap, uint32_t* __restrict__ cnt,
+                                                        uint32_t* __restrict__ missed, float* __restrict__ out_medians) {
+    __shared__ uint32_t s_h[2][NB];
+    __shared__ uint32_t s_prefix[2], s_rank[2];
+    const int f = blockIdx.x, tid = threadIdx.x;
+    const Bracket b = br[f];
+    if (tid == 0) cnt[f] = b.valid;
+    if (b.valid == 0) {
+        if (tid == 0) out_medians[f] = 0.0f;
+        return;
+    }
+    const uint32_t want[2] = {(b.valid - 1) / 2, b.valid / 2};
+    uint32_t key[2] = {0u, 0u};
+    bool search = false, miss = b.inside > cap;
+    for (int t = 0; t < 2; ++t) {
+        const uint32_t r = want[t] - b.below;  // wraps below the bracket: past every count
+        if (want[t] < b.below) miss = true;
+        else if (r < b.eq_lo) key[t] = b.lo;
+        else if (r - b.eq_lo < b.inside) search = true;
+        else if (r - b.eq_lo - b.inside < b.eq_hi) key[t] = b.hi;
+        else miss = true;
+    }
+    if (miss) {
+        if (tid == 0) *missed = 1;
+        return;
+    }
+    if (search) {
+        if (tid < 2) {
+            s_prefix[tid] = 0;
+            // a rank outside the list is clamped into it and its answer not used
+            const uint32_t r = want[tid] - b.below;
+            s_rank[tid] = r < b.eq_lo ? 0u : min(r - b.eq_lo, b.inside - 1);
+        }
+        const uint32_t* l = lists + (size_t)f * cap;
+        // digits of the distance from lo: the keys' common high bits would send
+        // every key of a pass to one counter
+        const int bits = 32 - __clz(b.hi - b.lo), passes = (bits + 7) / 8, width = (bits + passes - 1) / passes;
+        for (int shift = (passes - 1) * width; shift >= 0; shift -= width) {
+            if (tid < 2 * NB) (&s_h[0][0])[tid] = 0;
+            __syncthreads();
+            const uint32_t p0 = s_prefix[0], p1 = s_prefix[1];
+            for (uint32_t i = tid; i < b.inside; i += 1024) {
+                const uint32_t k = l[i] - b.lo, top = shift + width >= 32 ? 0u : k >> (shift + width),
+                               d = (k >> shift) & ((1u << width) - 1u);
+                if (top == p0) atomicAdd(&s_h[0][d], 1u);
+                if (top == p1) atomicAdd(&s_h[1][d], 1u);
+            }
+            __syncthreads();
+            if (tid < 2 * WAVE) {              // wave t: target t's digit, four digits a lane
+                const int t = tid / WAVE, lane = tid % WAVE;
+                uint32_t c[4], sum = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    c[q] = s_h[t][4 * lane + q];
+                    sum += c[q];
+                }
+                uint32_t run = wave_excl_scan<uint32_t>(sum, lane);
+                const uint32_t r = s_rank[t];
+                uint32_t d = 0, left = 0;
+                bool mine = false;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (r >= run && r < run + c[q]) {
+                        mine = true;
+                        d = 4 * lane + q;
+                        left = r - run;
+                    }
+                    run += c[q];
+                }
+                if (mine) {
+                    s_prefix[t] = (s_prefix[t] << width) | d;
+                    s_rank[t] = left;
+                }
+            }
+            __syncthreads();
+        }
+        for (int t = 0; t < 2; ++t) {
+            const uint32_t r = want[t] - b.below;
+            if (r >= b.eq_lo && r - b.eq_lo < b.inside) key[t] = b.lo + s_prefix[t];
+        }
+    }
+    if (tid == 0) {
+        const float a = kval(key[0]), c = kval(key[1]);
+        float med = (b.valid % 2) ? a : (a + c) / 2.0f;
+        if (isnan(med)) med = 0.0f;
+        out_medians[f] = med;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// medians over all rows: radix select of the two middle order statistics, run
+// where a bracket missed (a sample that is no random one); every kernel here
+// ends at once otherwise
+// ---------------------------------------------------------------------------
+
 // state[f][t] = {prefix, rank}: the ranks of the two middle order statistics.
-__global__ void k_select_init(const uint32_t* __restrict__ cnt, int F, uint32_t* __restrict__ state,
-                              uint32_t* __restrict__ hist) {
+__global__ void k_select_init(const uint32_t* __restrict__ missed, const uint32_t* __restrict__ cnt, int F,
+                              uint32_t* __restrict__ state, uint32_t* __restrict__ hist) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= F) return;
+    if (f >= F || !*missed) return;
     const uint32_t c = cnt[f];
     const uint32_t k1 = c == 0 ? 0 : (c % 2 ? (c - 1) / 2 : c / 2 - 1);
     const uint32_t k2 = c == 0 ? 0 : c / 2;
@@ -329,10 +688,11 @@ __global__ void k_select_init(const uint32_t* __restrict__ cnt, int F, uint32_t*
 }
 
 // Histogram of digit `shift` among keys whose higher bits equal each target's prefix.
-__global__ void __launch_bounds__(TB) k_select_hist(const float* __restrict__ X, int64_t ldx, int64_t n, int F,
-                                                    int shift, const uint32_t* __restrict__ state,
-                                                    uint32_t* __restrict__ hist) {
+__global__ void __launch_bounds__(TB) k_select_hist(const uint32_t* __restrict__ missed, const float* __restrict__ X,
+                                                    int64_t ldx, int64_t n, int F, int shift,
+                                                    const uint32_t* __restrict__ state, uint32_t* __restrict__ hist) {
     __shared__ uint32_t s_h[HT][2][NB];
+    if (!*missed) return;
     const int f0 = blockIdx.y * HT;
     for (int i = threadIdx.x; i < HT * 2 * NB; i += TB) (&s_h[0][0][0])[i] = 0;
     __syncthreads();
@@ -359,9 +719,10 @@ __global__ void __launch_bounds__(TB) k_select_hist(const float* __restrict__ X,
 }
 
 // Choose each target's digit; clear the histogram for the next pass.
-__global__ void k_select_step(int F, uint32_t* __restrict__ state, uint32_t* __restrict__ hist) {
+__global__ void k_select_step(const uint32_t* __restrict__ missed, int F, uint32_t* __restrict__ state,
+                              uint32_t* __restrict__ hist) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= F) return;
+    if (f >= F || !*missed) return;
     for (int t = 0; t < 2; ++t) {
         uint32_t* h = hist + (size_t)f * 2 * NB + (size_t)t * NB;
         uint32_t k = state[(size_t)f * 4 + 2 * t + 1];
@@ -378,10 +739,10 @@ __global__ void k_select_step(int F, uint32_t* __restrict__ state, uint32_t* __r
 
 // median = x_k (odd count) or float32 (x_k1 + x_k2) / 2 (even), 0 if no value
 // (np.nanmedian then np.where(isnan, 0, .), binning.py:32-33).
-__global__ void k_select_finish(const uint32_t* __restrict__ cnt, int F, const uint32_t* __restrict__ state,
-                                float* __restrict__ out_medians) {
+__global__ void k_select_finish(const uint32_t* __restrict__ missed, const uint32_t* __restrict__ cnt, int F,
+                                const uint32_t* __restrict__ state, float* __restrict__ out_medians) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= F) return;
+    if (f >= F || !*missed) return;
     const uint32_t c = cnt[f];
     float med = 0.0f;
     if (c > 0) {
@@ -572,27 +933,40 @@ int yabt_bin_fit(const float* X, int64_t ldx, int64_t n, int F, const int64_t* s
     const FitWs w = carve_fit((char*)workspace, m, F);
     if (workspace_bytes < w.bytes) return fail(-2, "yabt_bin_fit: workspace too small");
     // quantiles and scales of the sample (an empty sample is the column [0.0])
-    k_gather_keys<<<launch_grid(max(m, (int64_t)1) * F, TB, 8192), TB, 0, stream>>>(X, ldx, F, sample_rows, m,
-                                                                                     w.orig);
     if (m > 0) {
-        const hipError_t e =
-            hipMemcpyAsync(w.ka, w.orig, (size_t)F * m * sizeof(uint32_t), hipMemcpyDeviceToDevice, stream);
-        if (e != hipSuccess) return hip_fail(e, "yabt_bin_fit: key copy");
-        k_sort<<<F, SB, 0, stream>>>(w.ka, w.kb, m);
+        const dim3 tiles((unsigned)((m + 63) / 64), (unsigned)((F + 63) / 64));
+        k_gather_keys<<<tiles, TB, 0, stream>>>(X, ldx, F, sample_rows, m, w.orig);
+        if (m <= RC) {
+            k_sort_small<<<F, RT, 0, stream>>>(w.orig, w.ka, m);
+        } else {
+            const unsigned grid = (unsigned)(w.chunks * F);
+            const uint32_t* src = w.orig;
+            for (int pass = 0; pass < 4; ++pass) {
+                uint32_t* dst = pass & 1 ? w.ka : w.kb;
+                k_radix_count<<<grid, RT, 0, stream>>>(src, m, 8 * pass, w.chunks, w.dig);
+                k_radix_scan<<<F, 1024, 0, stream>>>(w.dig, w.chunks);
+                k_radix_scatter<<<grid, RT, 0, stream>>>(src, dst, m, 8 * pass, w.chunks, w.dig);
+                src = dst;
+            }
+        }
     }
-    k_quantiles<<<F, TB, 0, stream>>>(w.ka, w.orig, reinterpret_cast<float*>(w.kb), m, max_bins, out_edges, ld_edges,
-                                      out_nedges, out_scales);
+    const int whole = !sample_rows;            // the sample is all rows
+    k_quantiles<<<F, TB, 0, stream>>>(w.ka, m, max_bins, whole, out_edges, ld_edges, out_nedges, out_scales, out_medians,
+                                      w.need_std, w.br, w.missed);
+    k_std_scale<<<F, ST, 0, stream>>>(w.orig, reinterpret_cast<float*>(w.kb), m, w.need_std, out_scales);
+    if (whole) return launch_status("yabt_bin_fit launch");
     // medians over all n rows
-    const hipError_t e = hipMemsetAsync(w.cnt, 0, (size_t)F * sizeof(uint32_t), stream);
-    if (e != hipSuccess) return hip_fail(e, "yabt_bin_fit: clear");
+    const int fw = std::min(F, MT);
+    const dim3 pass((unsigned)launch_grid(n, MT / fw * 64, 2048), (unsigned)((F + fw - 1) / fw));
+    k_median_pass<<<pass, MT, 0, stream>>>(X, ldx, n, F, fw, w.br, w.kb, m);
+    k_median_finish<<<F, 1024, 0, stream>>>(w.br, w.kb, m, w.cnt, w.missed, out_medians);
     const dim3 grid((unsigned)launch_grid(max(n, (int64_t)1), TB / HT * 8, 1024), (unsigned)((F + HT - 1) / HT));
-    k_count_valid<<<grid, TB, 0, stream>>>(X, ldx, n, F, w.cnt);
-    k_select_init<<<(F + 63) / 64, 64, 0, stream>>>(w.cnt, F, w.sel_state, w.sel_hist);
+    k_select_init<<<(F + 63) / 64, 64, 0, stream>>>(w.missed, w.cnt, F, w.sel_state, w.sel_hist);
     for (int shift = 24; shift >= 0; shift -= 8) {
-        k_select_hist<<<grid, TB, 0, stream>>>(X, ldx, n, F, shift, w.sel_state, w.sel_hist);
-        k_select_step<<<(F + 63) / 64, 64, 0, stream>>>(F, w.sel_state, w.sel_hist);
+        k_select_hist<<<grid, TB, 0, stream>>>(w.missed, X, ldx, n, F, shift, w.sel_state, w.sel_hist);
+        k_select_step<<<(F + 63) / 64, 64, 0, stream>>>(w.missed, F, w.sel_state, w.sel_hist);
     }
-    k_select_finish<<<(F + 63) / 64, 64, 0, stream>>>(w.cnt, F, w.sel_state, out_medians);
+    k_select_finish<<<(F + 63) / 64, 64, 0, stream>>>(w.missed, w.cnt, F, w.sel_state, out_medians);
     return launch_status("yabt_bin_fit launch");
 }
 
