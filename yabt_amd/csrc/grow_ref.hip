@@ -108,6 +108,18 @@ __device__ __forceinline__ int job_of(const int32_t* off, int K, int64_t x) {
     return k;
 }
 
+// A tile's part of a sequential double sum, before the sum so far is known
+// (sum_apply).
+struct SumTry {
+    int l;                  // lowest set bit's exponent, LSB_NONE: all zero, LSB_BAD: inf or NaN among them
+    int64_t total;
+    float up, down;         // bounds of the largest and the most negative X_k, in units of 2^l
+};
+
+struct TileTry {                   // of g and h
+    SumTry c[2];
+};
+
 struct Ws {
     uint32_t* rows;                // RA arrays of rows_ld ids: depth % RA
     int64_t rows_ld;
@@ -125,6 +137,7 @@ struct Ws {
     int fgroup;                    // features bucketed per pass
     double* expl;                  // (KR, F, 3): sparse builder's explicit g, h sums, default-bin rows
     double* tot;                   // (KR, 2): sparse builder's node g, h sums
+    TileTry* tries;                // (n_tiles): sparse builder, per tile, its sums for the node totals
     float* hist;                   // (slots, 3, F, 256)
     int slots;                     // the root's and 2 per computed split
     int pend_cap;                  // computed splits, at most
@@ -165,6 +178,7 @@ Ws carve(char* base, int64_t n, int F, int max_leaves, bool sparse, int fgroup) 
     w.starts = c.take<uint16_t>((size_t)fgroup * (size_t)w.n_tiles * ST);
     w.expl = c.take<double>((size_t)KR * 3 * (size_t)F);
     w.tot = c.take<double>((size_t)KR * 2);
+    w.tries = sparse ? c.take<TileTry>((size_t)w.n_tiles) : nullptr;
     w.hist = c.take<float>((size_t)w.slots * 3 * F * NB);
     w.fsel = c.take<double>((size_t)2 * KR * F);
     w.fgain = c.take<double>((size_t)2 * KR * F);
@@ -367,25 +381,41 @@ __global__ void __launch_bounds__(RB) k_part_permute(const uint8_t* __restrict__
 // Dense (k_walk_chain_dense): the tile's g and h permuted into bucket order
 // in LDS, one thread per (bin, channel).
 //
-// Sparse builder (grow.c:68-107, default bins dbin; k_walk_chain<true>): the
+// Sparse builder (grow.c:68-107, default bins dbin; k_walk_chain_sparse): the
 // default bin gets no run; its thread instead adds, in double and in row
 // order, the tile's rows outside the default bin; block F adds the node's g
 // and h in double in row order; k_hist_default combines them.
 
 constexpr int SW = RB / WAVE;             // waves per sort / chain block
+// Blocks of a sparse sort that fill the device (3 a CU, twice over and more):
+// from so many on a block takes four features (child sorts 4.0 -> 1.9 ms at
+// 4M x 500), below one, for four times the blocks.
+constexpr int SORT_QUAD_BLOCKS = 2048;
 constexpr int SSUB = WT / SW;             // rows per wave per tile (sort)
 constexpr int SGR = SSUB / WAVE;          // 64-row groups per wave per tile (sort)
 constexpr int TPT = WT / RB;              // rows per thread per tile
 
-// Bin of the node's row at position x: row x for the root (rows[] is the
-// identity there, grow.c:289), rows[cs + x] of the children's array for a
-// built child.
+// Bins of a tile's tn rows (row t0 + x of the node) into s_bin: from the
+// feature-major column for the root (rows[] is the identity there,
+// grow.c:289; t0 % 16 == 0 and the column is padded to 16 rows), 16 rows a
+// thread with one load; by row id from the row-major copy else.
 template <bool ROOT>
-__device__ __forceinline__ uint32_t node_bin(const uint8_t* __restrict__ bins_fm, int64_t ld_fm,
-                                            const uint8_t* __restrict__ bins_rm, int64_t ld_rm,
-                                            const uint32_t* __restrict__ rows, int64_t cs, int f, int64_t x) {
-    if (ROOT) return bins_fm[(size_t)f * (size_t)ld_fm + (size_t)x];
-    return bins_rm[(size_t)rows[cs + x] * (size_t)ld_rm + f];
+__device__ __forceinline__ void tile_bins(const uint8_t* __restrict__ bins_fm, int64_t ld_fm,
+                                          const uint8_t* __restrict__ bins_rm, int64_t ld_rm,
+                                          const uint32_t* __restrict__ crow, int f, int64_t t0, int tn, uint8_t* s_bin) {
+    const int tid = threadIdx.x;
+    if (ROOT) {
+        static_assert(TPT == 16, "a thread's rows are one 16-byte load");
+        if (tid * 16 < tn)
+            *reinterpret_cast<uint4*>(s_bin + tid * 16) =
+                *reinterpret_cast<const uint4*>(bins_fm + (size_t)f * (size_t)ld_fm + (size_t)t0 + tid * 16);
+        return;
+    }
+#pragma unroll 2
+    for (int j = 0; j < TPT; ++j) {
+        const int x = j * RB + tid;
+        if (x < tn) s_bin[x] = bins_rm[(size_t)crow[t0 + x] * (size_t)ld_rm + f];
+    }
 }
 
 // Stable bucketing of one tile of one feature (block (f, t), t a tile of
@@ -396,50 +426,38 @@ __device__ __forceinline__ uint32_t node_bin(const uint8_t* __restrict__ bins_fm
 // total).  The lanes of a wave sharing a bin are found by an LDS atomic OR of
 // each lane's bit into s_peer[w][bin] (order-free), read back and cleared; a
 // row's rank is the number of those lanes below it plus the wave's running
-// count s_cnt[w][bin].  Sparse builder (dbin): the default bin gets no run,
-// and xperm lists the tile's other positions in row order.
-template <bool ROOT, bool SPARSE>
-__global__ void __launch_bounds__(RB, SPARSE ? 5 : 8) k_walk_sort(const uint8_t* __restrict__ bins_fm, int64_t ld_fm,
-                                                  const uint8_t* __restrict__ bins_rm, int64_t ld_rm,
-                                                  const uint32_t* __restrict__ rows, int64_t rows_ld,
-                                                  const Round* __restrict__ R, int fg0,
-                                                  const int32_t* __restrict__ dbin, uint16_t* __restrict__ perm,
-                                                  uint16_t* __restrict__ xperm, int64_t ld_perm,
-                                                  uint16_t* __restrict__ starts, int64_t n_tiles) {
-    __shared__ uint8_t s_bin[WT];
+// count s_cnt[w][bin].
+template <bool ROOT>
+__global__ void __launch_bounds__(RB, 8) k_walk_sort(const uint8_t* __restrict__ bins_fm, int64_t ld_fm,
+                                                     const uint8_t* __restrict__ bins_rm, int64_t ld_rm,
+                                                     const uint32_t* __restrict__ rows, int64_t rows_ld,
+                                                     const Round* __restrict__ R, int fg0,
+                                                     uint16_t* __restrict__ perm, int64_t ld_perm,
+                                                     uint16_t* __restrict__ starts, int64_t n_tiles) {
+    __shared__ __align__(16) uint8_t s_bin[WT];
     __shared__ uint64_t s_peer[SW][NB];            // once the tile is ranked: its bucketed positions
     __shared__ uint32_t s_cnt[SW][NB];
-    __shared__ uint16_t s_xperm[SPARSE ? WT : 1];
     static_assert(sizeof(s_peer) == WT * sizeof(uint16_t), "the bucketed positions fill the peer masks' space");
     uint16_t* s_perm = reinterpret_cast<uint16_t*>(&s_peer[0][0]);
     __shared__ uint32_t s_scan[SW];
-    __shared__ uint32_t s_xoff[SW + 1];
     const int fl = blockIdx.x, f = fg0 + fl;       // buffers by group position, bins by feature
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
-    const int df = SPARSE ? dbin[f] : -1;
     const int K = R->K;
     for (int64_t t = blockIdx.y; t < R->toff[K]; t += gridDim.y) {
     const int kj = job_of(R->toff, K, t);
     const Job& J = R->job[kj];
-    const int64_t cs = J.cs, m = J.ce - J.cs;
+    const int64_t m = J.ce - J.cs;
     const int64_t t0 = (t - R->toff[kj]) * WT;      // the tile's first row in the child
     if (t0 >= m) continue;                          // uniform across the block
-    const uint32_t* crow = rows + (size_t)J.dst * (size_t)rows_ld;
     const int tn = (int)min((int64_t)WT, m - t0);
     for (int i = tid; i < SW * NB; i += RB) {
         (&s_cnt[0][0])[i] = 0;
         (&s_peer[0][0])[i] = 0;
     }
-#pragma unroll 2
-    for (int j = 0; j < TPT; ++j) {
-        const int x = j * RB + tid;
-        if (x < tn) s_bin[x] = (uint8_t)node_bin<ROOT>(bins_fm, ld_fm, bins_rm, ld_rm, crow, cs, f, t0 + x);
-    }
+    tile_bins<ROOT>(bins_fm, ld_fm, bins_rm, ld_rm, rows + (size_t)J.dst * (size_t)rows_ld + J.cs, f, t0, tn, s_bin);
     __syncthreads();
-    // per group: the rank (bits 0-9), the sparse rank outside the default bin
-    // (bits 10-19) and the bin (bits 24-31) in one register
+    // per group: the rank (bits 0-9) and the bin (bits 24-31) in one register
     uint32_t pk[SGR];
-    uint32_t xrun = 0;
 #pragma unroll
     for (int q = 0; q < SGR; ++q) {
         const int x = w * SSUB + q * WAVE + lane;
@@ -455,18 +473,12 @@ __global__ void __launch_bounds__(RB, SPARSE ? 5 : 8) k_walk_sort(const uint8_t*
         if (v && r == 0) s_cnt[w][bin] = base + (uint32_t)__popcll(peers);
         __builtin_amdgcn_wave_barrier();
         pk[q] = (base + r) | (bin << 24);
-        if (SPARSE) {
-            const uint64_t xb = __ballot(v && (int)bin != df);
-            pk[q] |= (xrun + lane_prefix(xb)) << 10;
-            xrun += (uint32_t)__popcll(xb);
-        }
-        // packed here, not where it is used: otherwise its three parts stay
-        // live in registers of their own through the remaining groups
+        // packed here, not where it is used: otherwise its parts stay live in
+        // registers of their own through the remaining groups
         asm volatile("" : "+v"(pk[q]));
     }
-    if (SPARSE && lane == 0) s_xoff[w] = xrun;
     __syncthreads();
-    // bucket starts (sparse: no room for the default bin) and wave bases
+    // bucket starts and wave bases
     uint16_t* st_out = starts + ((size_t)fl * (size_t)n_tiles + (size_t)t) * ST;
     {
         const int b = tid;
@@ -477,7 +489,6 @@ __global__ void __launch_bounds__(RB, SPARSE ? 5 : 8) k_walk_sort(const uint8_t*
             c[u] = s_cnt[u][b];
             tb += c[u];
         }
-        if (SPARSE && b == df) tb = 0;
         uint32_t total;
         const uint32_t st = block_excl_scan<RB, uint32_t>(tb, s_scan, &total);
         st_out[b] = (uint16_t)st;
@@ -488,65 +499,177 @@ __global__ void __launch_bounds__(RB, SPARSE ? 5 : 8) k_walk_sort(const uint8_t*
             s_cnt[u][b] = run;
             run += c[u];
         }
-        if (SPARSE && tid == 0) {
-            uint32_t o = 0;
-#pragma unroll
-            for (int u = 0; u < SW; ++u) {
-                const uint32_t v = s_xoff[u];
-                s_xoff[u] = o;
-                o += v;
-            }
-            s_xoff[SW] = o;
-        }
     }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < SGR; ++q) {
         const int x = w * SSUB + q * WAVE + lane;
-        const uint32_t bin = pk[q] >> 24;
-        if (x < tn && (!SPARSE || (int)bin != df)) {
-            s_perm[s_cnt[w][bin] + (pk[q] & 1023u)] = (uint16_t)x;
-            if (SPARSE) s_xperm[s_xoff[w] + ((pk[q] >> 10) & 1023u)] = (uint16_t)x;
-        }
+        if (x < tn) s_perm[s_cnt[w][pk[q] >> 24] + (pk[q] & 1023u)] = (uint16_t)x;
     }
     __syncthreads();
-    const int total = SPARSE ? (int)s_xoff[SW] : tn;
     uint16_t* po = perm + (size_t)fl * (size_t)ld_perm + (size_t)t * WT;
-    for (int k = tid; k < total; k += RB) po[k] = s_perm[k];
-    if (SPARSE) {
-        uint16_t* xo = xperm + (size_t)fl * (size_t)ld_perm + (size_t)t * WT;
-        for (int k = tid; k < total; k += RB) xo[k] = s_xperm[k];
-    }
+    for (int k = tid; k < tn; k += RB) po[k] = s_perm[k];
     __syncthreads();
     }
 }
 
-// Sequential fp32 sums of the pairs s_gh[idx[k]], k in [lo, hi).
-__device__ __forceinline__ void run_f32(const float2* s_gh, const uint16_t* idx, uint32_t lo, uint32_t hi,
-                                        float& ag, float& ah) {
-    uint32_t k = lo;
-    for (; k + 8 <= hi; k += 8) {
-        uint32_t i[8];
+// The same for the sparse builder: the default bin's rows are left out first
+// (each thread lists the others of its 16 rows, in row order after one block
+// scan), and only the listed rows are ranked.  xperm lists their positions in
+// row order, perm the entries of xperm bin by bin; the default bin gets no
+// run.  4M x 500, 10% listed: the root's launch 1.8 ms where ranking all rows
+// took 8.5 ms.
+// QUAD: block x takes the four features 4 x .. 4 x + 3 (those of the group), whose
+// bytes of a row it gathers with one 4-byte load: the gathers touch a row's
+// line once per four features (1.9 ms of child sorts a tree against 4.0).
+template <bool ROOT, bool QUAD>
+__global__ void __launch_bounds__(RB, QUAD ? 3 : 5) k_walk_sort_sparse(const uint8_t* __restrict__ bins_fm, int64_t ld_fm,
+                                                            const uint8_t* __restrict__ bins_rm, int64_t ld_rm,
+                                                            const uint32_t* __restrict__ rows, int64_t rows_ld,
+                                                            const Round* __restrict__ R, int fg0, int nf,
+                                                            const int32_t* __restrict__ dbin, uint16_t* __restrict__ perm,
+                                                            uint16_t* __restrict__ xperm, int64_t ld_perm,
+                                                            uint16_t* __restrict__ starts, int64_t n_tiles) {
+    __shared__ __align__(16) uint8_t s_bin[WT];    // the tile's bins, then the listed rows'
+    __shared__ uint64_t s_peer[SW][NB];            // once ranked: the listed entries by bin
+    __shared__ uint32_t s_cnt[SW][NB];
+    __shared__ uint16_t s_x[WT];                   // the listed rows' positions
+    uint16_t* s_perm = reinterpret_cast<uint16_t*>(&s_peer[0][0]);
+    __shared__ uint32_t s_scan[SW];
+    __shared__ __align__(16) uint32_t s_quad[QUAD ? WT : 1];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
+    const int fq = QUAD ? 4 * (fg0 / 4 + (int)blockIdx.x) : 0;
+    const int K = R->K;
+    for (int64_t t = blockIdx.y; t < R->toff[K]; t += gridDim.y) {
+        const int kj = job_of(R->toff, K, t);
+        const Job& J = R->job[kj];
+        const int64_t m = J.ce - J.cs;
+        const int64_t t0 = (t - R->toff[kj]) * WT;      // the tile's first row in the child
+        if (t0 >= m) continue;                          // uniform across the block
+        const int tn = (int)min((int64_t)WT, m - t0);
+        if (QUAD) {
+            const uint32_t* crow = rows + (size_t)J.dst * (size_t)rows_ld + J.cs + t0;
+            constexpr int U = 8;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) i[j] = idx[k + j];
-        float2 p[8];
+            for (int j0 = 0; j0 < TPT; j0 += U) {
+                uint32_t r[U], b[U];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) p[j] = s_gh[i[j]];
+                for (int j = 0; j < U; ++j) r[j] = crow[min((j0 + j) * RB + tid, tn - 1)];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            ag += p[j].x;
-            ah += p[j].y;
+                for (int j = 0; j < U; ++j)
+                    b[j] = *reinterpret_cast<const uint32_t*>(bins_rm + (size_t)r[j] * (size_t)ld_rm + fq);
+#pragma unroll
+                for (int j = 0; j < U; ++j) s_quad[(j0 + j) * RB + tid] = b[j];
+            }
         }
-    }
-    for (; k < hi; ++k) {
-        const float2 p = s_gh[idx[k]];
-        ag += p.x;
-        ah += p.y;
+        for (int i4 = 0; i4 < (QUAD ? 4 : 1); ++i4) {
+            const int f = QUAD ? fq + i4 : fg0 + (int)blockIdx.x, fl = f - fg0;   // buffers by group position, bins by feature
+            if (fl < 0 || fl >= nf) continue;               // uniform across the block
+            const uint32_t df = (uint32_t)dbin[f];
+            for (int i = tid; i < SW * NB; i += RB) {
+                (&s_cnt[0][0])[i] = 0;
+                (&s_peer[0][0])[i] = 0;
+            }
+            if (!QUAD)
+                tile_bins<ROOT>(bins_fm, ld_fm, bins_rm, ld_rm, rows + (size_t)J.dst * (size_t)rows_ld + J.cs, f, t0, tn,
+                                s_bin);
+            __syncthreads();
+            // thread tid: rows 16 tid ..; which of them are listed
+            uint32_t bw[4];
+            if (QUAD) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint4 v = *reinterpret_cast<const uint4*>(s_quad + tid * 16 + 4 * q);
+                    bw[q] = ((v.x >> (8 * i4)) & 255u) | (((v.y >> (8 * i4)) & 255u) << 8) |
+                            (((v.z >> (8 * i4)) & 255u) << 16) | (((v.w >> (8 * i4)) & 255u) << 24);
+                }
+            } else {
+                const uint4 v = *reinterpret_cast<const uint4*>(s_bin + tid * 16);
+                bw[0] = v.x;
+                bw[1] = v.y;
+                bw[2] = v.z;
+                bw[3] = v.w;
+            }
+            const int mine = min(max(tn - tid * 16, 0), 16);
+            uint32_t listed = 0;
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                if (j < mine && ((bw[j >> 2] >> (8 * (j & 3))) & 255u) != df) listed |= 1u << j;
+            uint32_t nx;
+            uint32_t at = block_excl_scan<RB, uint32_t>((uint32_t)__popc(listed), s_scan, &nx);   // also: s_bin is read
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                if ((listed >> j) & 1u) {
+                    s_x[at] = (uint16_t)(tid * 16 + j);
+                    s_bin[at] = (uint8_t)(bw[j >> 2] >> (8 * (j & 3)));
+                    ++at;
+                }
+            __syncthreads();
+            // wave w ranks `groups` groups of 64 entries, the last wave's end short
+            const int groups = (int)((nx + SW * WAVE - 1) / (SW * WAVE));
+            uint32_t pk[SGR];
+#pragma unroll
+            for (int q = 0; q < SGR; ++q) {
+                pk[q] = 0;
+                if (q >= groups) continue;         // uniform
+                const uint32_t x = (uint32_t)((w * groups + q) * WAVE + lane);
+                const bool v = x < nx;
+                const uint32_t bin = v ? (uint32_t)s_bin[x] : 0u;
+                if (v) atomicOr(&s_peer[w][bin], 1ull << lane);
+                __builtin_amdgcn_wave_barrier();
+                const uint64_t peers = v ? s_peer[w][bin] : 0ull;
+                const uint32_t base = v ? s_cnt[w][bin] : 0u;
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t r = lane_prefix(peers);
+                if (v) s_peer[w][bin] = 0ull;
+                if (v && r == 0) s_cnt[w][bin] = base + (uint32_t)__popcll(peers);
+                __builtin_amdgcn_wave_barrier();
+                pk[q] = (base + r) | (bin << 24);
+                asm volatile("" : "+v"(pk[q]));
+            }
+            __syncthreads();
+            // bucket starts and wave bases
+            uint16_t* st_out = starts + ((size_t)fl * (size_t)n_tiles + (size_t)t) * ST;
+            {
+                const int b = tid;
+                uint32_t c[SW];
+                uint32_t tb = 0;
+#pragma unroll
+                for (int u = 0; u < SW; ++u) {
+                    c[u] = s_cnt[u][b];
+                    tb += c[u];
+                }
+                uint32_t total;
+                const uint32_t st = block_excl_scan<RB, uint32_t>(tb, s_scan, &total);
+                st_out[b] = (uint16_t)st;
+                if (b == NB - 1) st_out[NB] = (uint16_t)(st + tb);
+                uint32_t run = st;
+#pragma unroll
+                for (int u = 0; u < SW; ++u) {
+                    s_cnt[u][b] = run;
+                    run += c[u];
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < SGR; ++q) {
+                const uint32_t x = (uint32_t)((w * groups + q) * WAVE + lane);
+                if (q < groups && x < nx) s_perm[s_cnt[w][pk[q] >> 24] + (pk[q] & 1023u)] = (uint16_t)x;
+            }
+            __syncthreads();
+            uint16_t* po = perm + (size_t)fl * (size_t)ld_perm + (size_t)t * WT;
+            uint16_t* xo = xperm + (size_t)fl * (size_t)ld_perm + (size_t)t * WT;
+            for (uint32_t k = tid; k < nx; k += RB) {
+                po[k] = s_perm[k];
+                xo[k] = s_x[k];
+            }
+            __syncthreads();
+        }
     }
 }
 
 // The sequential double sum S <- RN(S + (double)x_k), k = 0 .. tn - 1 in
-// order, of each channel of the fp32 pairs s_gh[k] (cgrow's node totals,
+// order, of each channel of the tile's fp32 values (cgrow's node totals,
 // grow.c:85-97), computed by the whole block with the same result.  A step
 // rounds only when the exact partial sum does not fit a double's 53 bits,
 // and with fp32 addends that is rare (an addend far below |S|, or |S|
@@ -563,12 +686,8 @@ __device__ __forceinline__ void run_f32(const float2* s_gh, const uint16_t* idx,
 // part is below 2^53.  After TSE_TRIES restarts in one tile the remaining
 // elements are added one by one by one thread.  Every thread holds the same S.
 constexpr int TSE_TRIES = 8;
-// Element k of the sum: channel ch of s_gh[k], or of s_gh[idx[k]] with IDX.
-template <bool IDX>
-__device__ __forceinline__ float tse_x(const float2* s_gh, const uint16_t* idx, int ch, int k) {
-    const float2 p = s_gh[IDX ? (int)idx[k] : k];
-    return ch ? p.y : p.x;
-}
+// Element k of the sum: channel ch of the tile's staged values.
+__device__ __forceinline__ float tse_x(const float (*s_v)[WT], int ch, int k) { return s_v[ch][k]; }
 
 // The exponent of x's lowest set bit (x finite, nonzero).
 __device__ __forceinline__ int tse_lsb_exp(double x) {
@@ -583,9 +702,8 @@ __device__ __forceinline__ int tse_lsb_exp(double x) {
 // Both channels at once (g: c = 0, h: c = 1), so that they share the
 // block's passes and barriers; each channel restarts on its own.  s_wave:
 // 2 x RB / WAVE words, s_k, s_s, s_m: two each.
-template <bool IDX>
-__device__ void tile_sum_exact(const float2* s_gh, const uint16_t* idx, int tn, double (&S)[2], int64_t* s_wave,
-                               int* s_k, double* s_s, double* s_m) {
+__device__ void tile_sum_exact(const float (*s_v)[WT], int tn, double (&S)[2], int64_t* s_wave, int* s_k, double* s_s,
+                               double* s_m) {
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
     constexpr int NW = RB / WAVE;
     int k0[2] = {0, 0}, tries[2] = {0, 0};
@@ -600,7 +718,7 @@ __device__ void tile_sum_exact(const float2* s_gh, const uint16_t* idx, int tn, 
             if (act[c] && tries[c] >= TSE_TRIES) {
                 if (tid == c) {
                     double a = S[c];
-                    for (int k = k0[c]; k < tn; ++k) a += (double)tse_x<IDX>(s_gh, idx, c, k);
+                    for (int k = k0[c]; k < tn; ++k) a += (double)tse_x(s_v, c, k);
                     s_s[c] = a;
                 }
             }
@@ -622,7 +740,7 @@ __device__ void tile_sum_exact(const float2* s_gh, const uint16_t* idx, int tn, 
             kb[c] = k0[c] + tid * per;
             ke[c] = min(tn, kb[c] + per);
             if (act[c])
-                for (int k = kb[c]; k < ke[c]; ++k) am[c] += fabs((double)tse_x<IDX>(s_gh, idx, c, k));
+                for (int k = kb[c]; k < ke[c]; ++k) am[c] += fabs((double)tse_x(s_v, c, k));
 #pragma unroll
             for (int d = WAVE / 2; d > 0; d >>= 1) am[c] += __shfl_xor(am[c], d, WAVE);
         }
@@ -669,7 +787,7 @@ __device__ void tile_sum_exact(const float2* s_gh, const uint16_t* idx, int tn, 
             return t < ((uint64_t)1 << 53);
         };
         auto unit = [&](int c, int k, int64_t& r) -> bool {   // x_k / u, if an integer
-            const double v = (double)tse_x<IDX>(s_gh, idx, c, k) * sc[c];
+            const double v = (double)tse_x(s_v, c, k) * sc[c];
             if (v != rint(v) || fabs(v) >= 0x1p62) return false;
             r = (int64_t)v;
             return true;
@@ -732,7 +850,7 @@ __device__ void tile_sum_exact(const float2* s_gh, const uint16_t* idx, int tn, 
 #pragma unroll
         for (int c = 0; c < 2; ++c)
             if (act[c] && kf[c] != INT_MAX && kb[c] <= kf[c] && kf[c] < ke[c])   // cgrow's add of element kf
-                s_s[c] = (ldexp((double)Tbad[c], ue[c]) + Slo[c]) + (double)tse_x<IDX>(s_gh, idx, c, kf[c]);
+                s_s[c] = (ldexp((double)Tbad[c], ue[c]) + Slo[c]) + (double)tse_x(s_v, c, kf[c]);
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
@@ -750,58 +868,243 @@ __device__ void tile_sum_exact(const float2* s_gh, const uint16_t* idx, int tn, 
     }
 }
 
-// One tile of a chain block, TPT entries per thread, loaded a tile ahead.
-struct ChainTile {
-    float g[TPT], h[TPT];
-    uint32_t idx[TPT], xidx[TPT];
-    uint32_t st, st_end;
-};
+// The common case of that sum in one pass: no step of the tile rounds.  With
+// l the lowest set bit's exponent of any x_k, the partial sums X_k of the
+// x_k alone are integers of unit 2^l, so their total and extremes are exact in
+// int64; S + X_k is then a multiple of 2^min(l, lowest bit of S), and if the
+// extremes stay below 2^53 of those, every S + X_k is a double and cgrow's
+// sequence is S + total.  The extremes are taken as floats rounded up, so the
+// test errs on the safe side.
+constexpr int LSB_NONE = 4096, LSB_BAD = -4096;
 
-template <bool SPARSE>
-__device__ __forceinline__ void chain_load(ChainTile& c, const float* __restrict__ G, const float* __restrict__ H,
-                                           const uint16_t* __restrict__ pf, const uint16_t* __restrict__ xf,
-                                           const uint16_t* __restrict__ sf, bool totals, int64_t t, int64_t m) {
-    const int64_t t0 = t * WT;
-#pragma unroll
-    for (int j = 0; j < TPT; ++j) {
-        const int64_t x = t0 + j * RB + threadIdx.x;
-        if (x < m) {
-            c.g[j] = G[x];
-            c.h[j] = H[x];
-            if (!totals) {
-                c.idx[j] = pf[x];
-                if (SPARSE) c.xidx[j] = xf[x];
-            }
+// The exponent of x's lowest set bit.
+__device__ __forceinline__ int f32_lsb(float x) {
+    const uint32_t b = __float_as_uint(x) & 0x7fffffffu, e = b >> 23;
+    if (b == 0) return LSB_NONE;
+    if (e == 255) return LSB_BAD;
+    return max((int)e, 1) - 150 + __builtin_ctz((b & 0x7fffffu) | (e ? 0x800000u : 0u));
+}
+
+// One thread's elements [kb, ke): their sum and extremes in units of 2^l;
+// false if one is too large for the int64 sums.
+__device__ __forceinline__ bool sum_units(const float* s, int kb, int ke, int l, int64_t& sum, int64_t& mx, int64_t& mn) {
+    const double sc = ldexp(1.0, -l);
+    bool ok = true;
+    sum = mx = mn = 0;
+    for (int k = kb; k < ke; ++k) {
+        const double v = (double)s[k] * sc;    // an integer
+        ok = ok && fabs(v) < 0x1p49;           // 4096 of them stay below 2^61
+        sum += ok ? (int64_t)v : 0;
+        mx = max(mx, sum);
+        mn = min(mn, sum);
+    }
+    return ok;
+}
+
+__device__ __forceinline__ float round_up_f32(int64_t v) { return v > 0 ? (float)v * 1.000001f : 0.0f; }
+__device__ __forceinline__ float wave_max_pos(float v) { return __int_as_float(-wave_min_i32(-__float_as_int(v))); }
+
+// Whether the tile's sum is t.total added exactly; S is then updated.
+__device__ __forceinline__ bool sum_apply(const SumTry& t, double& S) {
+    if (t.l == LSB_NONE) return true;
+    if (t.l == LSB_BAD || !(fabs(S) < 0x1p900) || t.up >= 0x1p51f || t.down >= 0x1p51f) return false;
+    const double u = ldexp(1.0, t.l);
+    const int lm = S == 0.0 ? t.l : min(t.l, tse_lsb_exp(S));
+    const double far = fmax(fabs(S + (double)t.up * u), fabs(S - (double)t.down * u)) * (1.0 + 0x1p-40);
+    if (!(far < ldexp(1.0, lm + 53))) return false;
+    S += (double)t.total * u;
+    return true;
+}
+
+// S <- cgrow's sequential double sum of S and s[0 .. n - 1], by one wave.
+__device__ __forceinline__ void wave_sum_exact(const float* s, int n, double& S, int lane) {
+    const int per = ((n + WAVE - 1) / WAVE) | 1;   // odd: neighbouring lanes' reads on different banks
+    const int kb = min(n, lane * per), ke = min(n, kb + per);
+    SumTry t;
+    int l = LSB_NONE;
+    for (int k = kb; k < ke; ++k) l = min(l, f32_lsb(s[k]));
+    t.l = wave_min_i32(l);
+    if (t.l == LSB_NONE) return;
+    if (t.l != LSB_BAD) {
+        int64_t sum, mx, mn;
+        const bool ok = sum_units(s, kb, ke, t.l, sum, mx, mn);
+        if (__ballot(!ok)) {
+            t.l = LSB_BAD;
+        } else {
+            const int64_t incl = wave_incl_scan_i64(sum, lane), ex = incl - sum;
+            t.total = readlane64(incl, WAVE - 1);
+            t.up = wave_max_pos(round_up_f32(mx + ex));
+            t.down = wave_max_pos(round_up_f32(-(mn + ex)));
         }
     }
-    if (!totals) {
-        c.st = sf[(size_t)t * ST + threadIdx.x];
-        if (threadIdx.x == 0) c.st_end = sf[(size_t)t * ST + NB];
+    if (sum_apply(t, S)) return;
+    double a = S;                              // one by one; every lane does the same adds
+    int k = 0;
+    for (; k + 8 <= n; k += 8) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = s[k + j];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a += (double)v[j];
+    }
+    for (; k < n; ++k) a += (double)s[k];
+    S = a;
+}
+
+// Both channels' SumTry of every tile of the round's built children (block t),
+// for the node totals: they need S only when they are applied, tile by tile.
+
+__global__ void __launch_bounds__(RB) k_total_tries(const float* __restrict__ Gb, const float* __restrict__ Hb,
+                                                    const Round* __restrict__ R, TileTry* __restrict__ tries) {
+    __shared__ float s_v[2][WT];
+    __shared__ int64_t s_wave[2][RB / WAVE];
+    __shared__ int s_l[2], s_bad[2];
+    __shared__ uint32_t s_far[2][2];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
+    for (int64_t t = blockIdx.x; t < R->toff[R->K]; t += gridDim.x) {
+        const int kj = job_of(R->toff, R->K, t);
+        const Job& J = R->job[kj];
+        const int64_t t0 = J.cs + (t - R->toff[kj]) * WT;
+        if (t0 >= J.ce) continue;              // uniform across the block
+        const int tn = (int)min((int64_t)WT, J.ce - t0);
+#pragma unroll
+        for (int j = 0; j < TPT; ++j) {        // rows past the end read the last one
+            const int64_t x = t0 + min(j * RB + tid, tn - 1);
+            s_v[0][j * RB + tid] = Gb[x];
+            s_v[1][j * RB + tid] = Hb[x];
+        }
+        if (tid < 2) {
+            s_l[tid] = LSB_NONE;
+            s_bad[tid] = 0;
+            s_far[tid][0] = s_far[tid][1] = 0;
+        }
+        __syncthreads();
+        const int per = ((tn + RB - 1) / RB) | 1, kb = min(tn, tid * per), ke = min(tn, kb + per);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            int l = LSB_NONE;
+            for (int k = kb; k < ke; ++k) l = min(l, f32_lsb(s_v[c][k]));
+            l = wave_min_i32(l);
+            if (lane == 0) atomicMin(&s_l[c], l);
+        }
+        __syncthreads();
+        int64_t ex[2], mx[2], mn[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            int64_t sum = 0;
+            mx[c] = mn[c] = 0;
+            bool ok = true;
+            if (s_l[c] != LSB_NONE && s_l[c] != LSB_BAD) ok = sum_units(s_v[c], kb, ke, s_l[c], sum, mx[c], mn[c]);
+            const int64_t incl = wave_incl_scan_i64(sum, lane);
+            ex[c] = incl - sum;
+            if (lane == WAVE - 1) s_wave[c][w] = incl;
+            if (__ballot(!ok) && lane == 0) s_bad[c] = 1;   // too large for the int64 sums
+        }
+        __syncthreads();
+        int64_t tot[2] = {0, 0};
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            int64_t off = 0;
+#pragma unroll
+            for (int i = 0; i < RB / WAVE; ++i) {
+                if (i < w) off += s_wave[c][i];
+                tot[c] += s_wave[c][i];
+            }
+            const float up = wave_max_pos(round_up_f32(mx[c] + ex[c] + off));
+            const float down = wave_max_pos(round_up_f32(-(mn[c] + ex[c] + off)));
+            if (lane == 0) {
+                atomicMax(&s_far[c][0], __float_as_uint(up));
+                atomicMax(&s_far[c][1], __float_as_uint(down));
+            }
+        }
+        __syncthreads();
+        if (tid < 2) {
+            SumTry r;
+            r.l = s_bad[tid] ? LSB_BAD : s_l[tid];
+            r.total = tid ? tot[1] : tot[0];
+            r.up = __uint_as_float(s_far[tid][0]);
+            r.down = __uint_as_float(s_far[tid][1]);
+            tries[t].c[tid] = r;
+        }
+        __syncthreads();
     }
 }
 
-// The chains with default bins (block f, thread b = bin; SPARSE; dense
-// chains run in k_walk_chain_dense): the node's tiles in order, each tile's
-// g, h and bucketed positions staged in LDS, bin b's run added in fp32 in row
-// order (grow.c:55-59); the count cell is cgrow's chain of 1.0f adds, which
-// is min(count, 2^24) exactly.  The default bin's thread adds the tile's
-// other rows in double in row order (xperm), and block F adds the node's g
-// and h in double in row order (grow.c:85-97); k_hist_default combines them.
-// G, H hold the node's g, h by position.
-// Block (f, k): job k's built child (its tiles R->toff[k] ..); G, H hold the
-// g, h of the child's rows at their positions.
-template <bool SPARSE>
-__global__ void __launch_bounds__(RB) k_walk_chain(const float* __restrict__ Gb, const float* __restrict__ Hb,
-                                                   const Round* __restrict__ R, int F, int fg0, int nf,
-                                                   const int32_t* __restrict__ dbin,
-                                                   const uint16_t* __restrict__ perm,
-                                                   const uint16_t* __restrict__ xperm, int64_t ld_perm,
-                                                   const uint16_t* __restrict__ starts, int64_t n_tiles,
-                                                   float* __restrict__ hist_base, size_t hsz,
-                                                   double* __restrict__ eout_b, double* __restrict__ tot_b) {
-    __shared__ __align__(16) float2 s_gh[WT];
+// The node's g and h in double in row order, by one block: the tiles' sums
+// applied one after the other; a tile in which a step may round is summed by
+// tile_sum_exact.  Every thread holds the same S.
+__device__ void node_totals(const float* __restrict__ G, const float* __restrict__ H, int64_t m,
+                            const TileTry* __restrict__ tries, float (*s_v)[WT], double (&S)[2], int64_t* s_wave, int* s_k,
+                            double* s_s, double* s_m) {
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+    const int64_t tiles = (m + WT - 1) / WT;
+    for (int64_t b = 0; b < tiles; b += WAVE) {    // lane i: tile b + i's
+        const TileTry mine = tries[min(b + lane, tiles - 1)];
+        const int nt = (int)min((int64_t)WAVE, tiles - b);
+        for (int i = 0; i < nt; ++i) {
+            double T[2] = {S[0], S[1]};
+            bool ok = true;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                SumTry t;
+                t.l = __builtin_amdgcn_readlane(mine.c[c].l, i);
+                t.total = readlane64(mine.c[c].total, i);
+                t.up = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.c[c].up), i));
+                t.down = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.c[c].down), i));
+                ok = sum_apply(t, T[c]) && ok;
+            }
+            if (ok) {                          // the same in every wave
+                S[0] = T[0];
+                S[1] = T[1];
+                continue;
+            }
+            const int64_t t0 = (b + i) * WT;
+            const int tn = (int)min((int64_t)WT, m - t0);
+            for (int x = tid; x < tn; x += RB) {
+                s_v[0][x] = G[t0 + x];
+                s_v[1][x] = H[t0 + x];
+            }
+            __syncthreads();
+            tile_sum_exact(s_v, tn, S, s_wave, s_k, s_s, s_m);
+            __syncthreads();
+        }
+    }
+}
+
+// The chains with default bins (dense chains run in k_walk_chain_dense).
+// Block (f, k): feature f of job k's built child, its tiles in order.  Of a
+// tile only the rows outside the default bin are touched: their positions
+// (xperm) two tiles ahead, their g and h one tile ahead, into LDS in row
+// order.  Waves 0 and 1 then add g and h in double in row order (the
+// default bin's E, grow.c:85-97); waves 2 and 3 add each bin's run (perm:
+// places in that order, bin by bin) in fp32 in row order (grow.c:55-59), two
+// bins a lane.  The count cell is cgrow's chain of 1.0f adds, min(count,
+// 2^24).  Block nf of the first group adds the node's g and h in double in
+// row order; k_hist_default combines them.
+//
+// Bound by the tile's steps, one after the other by definition: 3.5 us a
+// tile at 4M x 500, 10% outside the default bin (root launch 3.4 ms).  With
+// every row's g, h and both lists' full tiles loaded (48 KB a tile and
+// feature against ~5) and the sums by the whole block with eight or more
+// barriers a tile it took 18.6 us (18.2 ms).  Rows two tiles ahead: no gain at
+// the root (3.7 ms) and fewer blocks a CU for the children.
+struct SparseTile {
+    float g[TPT], h[TPT];
+    uint32_t idx[TPT];
+    uint32_t st, st_end;
+};
+
+__global__ void __launch_bounds__(RB) k_walk_chain_sparse(const float* __restrict__ Gb, const float* __restrict__ Hb,
+                                                          const Round* __restrict__ R, int F, int fg0, int nf,
+                                                          const int32_t* __restrict__ dbin,
+                                                          const uint16_t* __restrict__ perm,
+                                                          const uint16_t* __restrict__ xperm, int64_t ld_perm,
+                                                          const uint16_t* __restrict__ starts, int64_t n_tiles,
+                                                          float* __restrict__ hist_base, size_t hsz,
+                                                          const TileTry* __restrict__ tries,
+                                                          double* __restrict__ eout_b, double* __restrict__ tot_b) {
+    __shared__ float s_v[2][WT];
     __shared__ uint16_t s_idx[WT];
-    __shared__ uint16_t s_xidx[SPARSE ? WT : 1];
     __shared__ uint16_t s_st[ST];
     __shared__ int64_t s_tw[2 * (RB / WAVE)];         // the totals block's scans
     __shared__ int s_tk[2];
@@ -812,82 +1115,122 @@ __global__ void __launch_bounds__(RB) k_walk_chain(const float* __restrict__ Gb,
     const int64_t tile0 = R->toff[kj];
     const float* G = Gb + J.cs;
     const float* H = Hb + J.cs;
-    double* eout = eout_b + (size_t)kj * 3 * F;
-    double* tot = tot_b + (size_t)kj * 2;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
     const int fl = blockIdx.x, f = fg0 + fl;       // buffers by group position, cells by feature
-    const bool totals = SPARSE && fl == nf;        // the extra block of the first group
-    const int df = (SPARSE && !totals) ? dbin[f] : -1;
-    const size_t fo = (size_t)(totals ? 0 : fl);
-    const uint16_t* pf = perm + fo * (size_t)ld_perm + (size_t)tile0 * WT;
-    const uint16_t* xf = SPARSE ? xperm + fo * (size_t)ld_perm + (size_t)tile0 * WT : nullptr;
-    const uint16_t* sf = starts + (fo * (size_t)n_tiles + (size_t)tile0) * ST;
-    float ag = 0.0f, ah = 0.0f;
-    double eg = 0.0, eh = 0.0;
-    int64_t cnt = 0;
-    ChainTile nxt;
-    if (m > 0) chain_load<SPARSE>(nxt, G, H, pf, xf, sf, totals, 0, m);
-    for (int64_t t = 0, t0 = 0; t0 < m; ++t, t0 += WT) {
-        const int tn = (int)min((int64_t)WT, m - t0);
-#pragma unroll
-        for (int j = 0; j < TPT; ++j) {
-            const int x = j * RB + tid;
-            if (x < tn) {
-                s_gh[x] = make_float2(nxt.g[j], nxt.h[j]);
-                if (!totals) {
-                    s_idx[x] = (uint16_t)nxt.idx[j];
-                    if (SPARSE) s_xidx[x] = (uint16_t)nxt.xidx[j];
-                }
-            }
-        }
-        if (!totals) {
-            s_st[tid] = (uint16_t)nxt.st;
-            if (tid == 0) s_st[NB] = (uint16_t)nxt.st_end;
-        }
-        __syncthreads();
-        if (t0 + WT < m) chain_load<SPARSE>(nxt, G, H, pf, xf, sf, totals, t + 1, m);
-        if (totals) {
-            // the node's g and h in double in row order, by the whole block
-            double S2[2] = {eg, eh};
-            tile_sum_exact<false>(s_gh, nullptr, tn, S2, s_tw, s_tk, s_ts, s_tm);
-            eg = S2[0];
-            eh = S2[1];
-        } else {
-            if (SPARSE && tid == df) {
-                cnt += (int64_t)tn - s_st[NB];
-            } else {
-                const uint32_t lo = s_st[tid], hi = s_st[tid + 1];
-                run_f32(s_gh, s_idx, lo, hi, ag, ah);
-                cnt += hi - lo;
-            }
-            if (SPARSE) {
-                // the tile's rows outside the default bin (xidx, in row
-                // order), their g and h in double, by the whole block
-                double S2[2] = {eg, eh};
-                tile_sum_exact<true>(s_gh, s_xidx, (int)s_st[NB], S2, s_tw, s_tk, s_ts, s_tm);
-                eg = S2[0];
-                eh = S2[1];
-            }
-        }
-        __syncthreads();
-    }
-    if (totals) {
+    if (fl == nf) {                                // the node totals
+        double S2[2] = {0.0, 0.0};
+        node_totals(G, H, m, tries + tile0, s_v, S2, s_tw, s_tk, s_ts, s_tm);
         if (tid == 0) {
-            tot[0] = eg;
-            tot[1] = eh;
+            tot_b[(size_t)kj * 2] = S2[0];
+            tot_b[(size_t)kj * 2 + 1] = S2[1];
         }
         return;
     }
+    const int df = dbin[f];
+    const uint16_t* pf = perm + (size_t)fl * (size_t)ld_perm + (size_t)tile0 * WT;
+    const uint16_t* xf = xperm + (size_t)fl * (size_t)ld_perm + (size_t)tile0 * WT;
+    const uint16_t* sf = starts + ((size_t)fl * (size_t)n_tiles + (size_t)tile0) * ST;
+    const int64_t tiles = (m + WT - 1) / WT;
+    // entries of tile t outside the default bin (0 past the last tile)
+    const auto entries = [&](int64_t t) { return t < tiles ? (int)sf[(size_t)t * ST + NB] : 0; };
+    uint32_t xp[TPT];
+    const auto load_pos = [&](int64_t t, int nx) {
+#pragma unroll
+        for (int j = 0; j < TPT; ++j)
+            if (j * RB < nx) xp[j] = xf[(size_t)t * WT + min(j * RB + tid, nx - 1)];
+    };
+    SparseTile nxt;
+    const auto load_rows = [&](int64_t t, int nx) {
+        const int64_t t0 = t * WT;
+#pragma unroll
+        for (int j = 0; j < TPT; ++j)
+            if (j * RB < nx) {
+                nxt.g[j] = G[t0 + xp[j]];
+                nxt.h[j] = H[t0 + xp[j]];
+                nxt.idx[j] = pf[t0 + min(j * RB + tid, nx - 1)];
+            }
+        nxt.st = sf[(size_t)t * ST + tid];
+        nxt.st_end = sf[(size_t)t * ST + NB];
+    };
+    double E = 0.0;                                // wave 0: g's, wave 1: h's
+    float ag[2] = {0.0f, 0.0f}, ah[2] = {0.0f, 0.0f};
+    int64_t cnt[2] = {0, 0}, other = 0;
+    int nx = __builtin_amdgcn_readfirstlane(entries(0)), nx1 = __builtin_amdgcn_readfirstlane(entries(1));
+    int nx2 = entries(2);
+    if (m > 0) {
+        load_pos(0, nx);
+        load_rows(0, nx);
+        load_pos(1, nx1);
+    }
+    for (int64_t t = 0; t < tiles; ++t) {
+        const int tn = (int)min((int64_t)WT, m - t * WT);
+#pragma unroll
+        for (int j = 0; j < TPT; ++j)
+            if (j * RB < nx) {                     // places past nx hold copies that nothing reads
+                s_v[0][j * RB + tid] = nxt.g[j];
+                s_v[1][j * RB + tid] = nxt.h[j];
+                s_idx[j * RB + tid] = (uint16_t)nxt.idx[j];
+            }
+        s_st[tid] = (uint16_t)nxt.st;
+        if (tid == 0) s_st[NB] = (uint16_t)nxt.st_end;
+        __syncthreads();
+        const int nx3 = entries(t + 3);
+        nx2 = __builtin_amdgcn_readfirstlane(nx2);
+        if (t + 1 < tiles) load_rows(t + 1, nx1);
+        load_pos(t + 2, nx2);
+        if (w < 2) {
+            wave_sum_exact(s_v[w], nx, E, lane);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int b = (w - 2) * WAVE + lane + c * (NB / 2);
+                uint32_t k = s_st[b];
+                const uint32_t hi = s_st[b + 1];
+                cnt[c] += hi - k;
+                for (; k + 4 <= hi; k += 4) {
+                    uint32_t i[4];
+                    float vg[4], vh[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) i[u] = s_idx[k + u];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        vg[u] = s_v[0][i[u]];
+                        vh[u] = s_v[1][i[u]];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        ag[c] += vg[u];
+                        ah[c] += vh[u];
+                    }
+                }
+                for (; k < hi; ++k) {
+                    const uint32_t i = s_idx[k];
+                    ag[c] += s_v[0][i];
+                    ah[c] += s_v[1][i];
+                }
+            }
+        }
+        other += tn - nx;                          // rows in the default bin
+        __syncthreads();
+        nx = nx1;
+        nx1 = nx2;
+        nx2 = nx3;
+    }
     const int slot = J.build_left ? J.slot_l : J.slot_r;
     float* hist = hist_base + (size_t)slot * hsz;
-    if (SPARSE && tid == df) {
-        eout[3 * (size_t)f] = eg;
-        eout[3 * (size_t)f + 1] = eh;
-        eout[3 * (size_t)f + 2] = (double)cnt;
-    } else {
-        hist[(size_t)0 * F * NB + (size_t)f * NB + tid] = ag;
-        hist[(size_t)1 * F * NB + (size_t)f * NB + tid] = ah;
-        hist[(size_t)2 * F * NB + (size_t)f * NB + tid] = (float)min(cnt, (int64_t)1 << 24);
+    double* eout = eout_b + (size_t)kj * 3 * F + 3 * (size_t)f;
+    if (w < 2) {
+        if (lane == 0) eout[w] = E;
+        if (w == 0 && lane == 0) eout[2] = (double)other;
+        return;
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int b = (w - 2) * WAVE + lane + c * (NB / 2);
+        if (b == df) continue;                     // k_hist_default writes it
+        hist[(size_t)0 * F * NB + (size_t)f * NB + b] = ag[c];
+        hist[(size_t)1 * F * NB + (size_t)f * NB + b] = ah[c];
+        hist[(size_t)2 * F * NB + (size_t)f * NB + b] = (float)min(cnt[c], (int64_t)1 << 24);
     }
 }
 
@@ -1834,20 +2177,26 @@ struct Grower {
         for (int fg0 = 0; fg0 < F; fg0 += w.fgroup) {
             const int nf = min(w.fgroup, F - fg0);
             const dim3 sgrid((unsigned)nf, ty);
-#define YABT_SORT(ROOT, SPARSE)                                                                             \
-    k_walk_sort<ROOT, SPARSE><<<sgrid, RB, 0, st>>>(bins_fm, ld_fm, bins_rm, ld_rm, w.rows, w.rows_ld, w.round, \
-                                                    fg0, dbin, w.perm, w.xperm, w.ld_perm, w.starts, w.n_tiles)
-            if (root) {
-                if (dbin) YABT_SORT(true, true); else YABT_SORT(true, false);
+            if (dbin) {
+                // four features a block where that still fills the device
+                const int quads = (fg0 + nf - 1) / 4 - fg0 / 4 + 1;
+                const bool quad = !root && (int64_t)quads * tiles >= SORT_QUAD_BLOCKS;
+                auto sort = root ? k_walk_sort_sparse<true, false>
+                                 : (quad ? k_walk_sort_sparse<false, true> : k_walk_sort_sparse<false, false>);
+                sort<<<quad ? dim3((unsigned)quads, ty) : sgrid, RB, 0, st>>>(
+                    bins_fm, ld_fm, bins_rm, ld_rm, w.rows, w.rows_ld, w.round, fg0, nf, dbin, w.perm, w.xperm, w.ld_perm,
+                    w.starts, w.n_tiles);
+                if (fg0 == 0) k_total_tries<<<ty, RB, 0, st>>>(G, H, w.round, w.tries);
             } else {
-                if (dbin) YABT_SORT(false, true); else YABT_SORT(false, false);
+                auto sort = root ? k_walk_sort<true> : k_walk_sort<false>;
+                sort<<<sgrid, RB, 0, st>>>(bins_fm, ld_fm, bins_rm, ld_rm, w.rows, w.rows_ld, w.round, fg0, w.perm,
+                                           w.ld_perm, w.starts, w.n_tiles);
             }
-#undef YABT_SORT
             // the sparse builder's node totals: one more block with the first group
             const dim3 cgrid((unsigned)nf + (dbin && fg0 == 0 ? 1u : 0u), (unsigned)K);
             if (dbin)
-                k_walk_chain<true><<<cgrid, RB, 0, st>>>(G, H, w.round, F, fg0, nf, dbin, w.perm, w.xperm, w.ld_perm,
-                                                         w.starts, w.n_tiles, w.hist, hsz, w.expl, w.tot);
+                k_walk_chain_sparse<<<cgrid, RB, 0, st>>>(G, H, w.round, F, fg0, nf, dbin, w.perm, w.xperm, w.ld_perm,
+                                                          w.starts, w.n_tiles, w.hist, hsz, w.tries, w.expl, w.tot);
             else
                 k_walk_chain_dense<<<cgrid, CB, 0, st>>>(G, H, w.round, F, fg0, w.perm, w.ld_perm, w.starts,
                                                          w.n_tiles, w.hist, hsz);
