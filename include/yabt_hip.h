@@ -377,7 +377,7 @@ size_t yabt_grow_ref_workspace_min_bytes(int64_t n, int F, int max_leaves, int s
  * which computes up to 16 splits per round (planned by running the table
  * ahead through the splits already computed) and commits them in cgrow's
  * order: one device round trip per round.  root_order (NULL: the root is
- * bucketed in the call): the rank table yabt_ref_root_order made for these
+ * bucketed in the call): the root table yabt_ref_root_order made for these
  * bins_fm, n and F, which the dense builder's root then reads instead of
  * bucketing its rows again (the sparse builder ignores it).  The call returns
  * after the stream has finished (it synchronises `stream`).  Requires
@@ -391,13 +391,13 @@ int yabt_grow_ref(const uint8_t *bins_fm, int64_t ld_fm, const uint8_t *bins_rm,
                   float *out_value, int64_t *out_depth, int64_t *out_leaf_of_row, int64_t *out_rows,
                   int32_t *out_n_nodes, yabt_stream_t stream);
 
-/* Bytes of the root rank table of yabt_ref_root_order for n rows, F features
+/* Bytes of the root table of yabt_ref_root_order for n rows, F features
  * (0: bad sizes). */
 size_t yabt_ref_root_order_bytes(int64_t n, int F);
 
-/* The root rank table of yabt_grow_ref's dense builder, once per fit: for
- * every feature and every 4096-row tile of rows 0 .. n - 1, each row's rank
- * among the tile's rows in its bin (row order), the tile's bin starts, its
+/* The root table of yabt_grow_ref's dense builder, once per fit: for
+ * every feature and every 4096-row tile of rows 0 .. n - 1, the tile's rows
+ * bucketed by bin (row order inside a bin), the tile's bin starts, its
  * longest run and its largest bin --
  * the bucketing of cgrow's row-order histogram chains (yabt/_cgrow/grow.c:
  * 37-62) of the root, which is the same for every tree grown on these bins.
@@ -410,7 +410,7 @@ int yabt_ref_root_order(const uint8_t *bins_fm, int64_t ld_fm, int64_t n, int F,
 /* The reference-arithmetic root histogram alone: out (3, F, 256) float32 =
  * cgrow's dense build_hist over rows 0 .. n - 1 (yabt/_cgrow/grow.c:37-62):
  * per (feature, bin) the fp32 sums of g, of h and of 1.0f in row order, from
- * the rank table yabt_ref_root_order made for these bins (root_order_bytes:
+ * the root table yabt_ref_root_order made for these bins (root_order_bytes:
  * its size).  Replaces build_hist for the root node. */
 int yabt_ref_root_hist(const uint8_t *bins_fm, int64_t ld_fm, const float *grad, const float *hess, int64_t n,
                        int F, const void *root_order, size_t root_order_bytes, float *out, yabt_stream_t stream);

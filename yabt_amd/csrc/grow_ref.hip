@@ -378,7 +378,7 @@ __global__ void __launch_bounds__(RB) k_part_permute(const uint8_t* __restrict__
 // parallel over the whole device; a chain kernel then runs one block per
 // (feature, split) over the tiles in order, adding bin b's run of each tile
 // to its fp32 accumulators, so every cell is cgrow's sequential sum.
-// Dense (k_walk_chain_dense): the tile's g and h permuted into bucket order
+// Dense (k_tile_chain, k_walk_chain_dense): the tile's g and h permuted into bucket order
 // in LDS, one thread per (bin, channel).
 //
 // Sparse builder (grow.c:68-107, default bins dbin; k_walk_chain_sparse): the
@@ -1071,7 +1071,7 @@ __device__ void node_totals(const float* __restrict__ G, const float* __restrict
     }
 }
 
-// The chains with default bins (dense chains run in k_walk_chain_dense).
+// The chains with default bins (dense chains: k_tile_chain, k_walk_chain_dense).
 // Block (f, k): feature f of job k's built child, its tiles in order.  Of a
 // tile only the rows outside the default bin are touched: their positions
 // (xperm) two tiles ahead, their g and h one tile ahead, into LDS in row
@@ -1234,6 +1234,10 @@ __global__ void __launch_bounds__(RB) k_walk_chain_sparse(const float* __restric
     }
 }
 
+constexpr int CB = 2 * RB;           // adding threads of a chain block (a bin's g chain, then its h chain), and loading ones
+constexpr int CPT = WT / CB;         // positions per loading thread and tile
+constexpr int CQ = CPT / 4;
+
 // Sequential fp32 sum of s[k], k in [lo, hi) (hi <= WT): blocks of 16 read 8
 // ahead of the adds, so that a long run (a bin that holds most of a tile, as
 // the features on a node's path do) waits about one LDS latency per 16
@@ -1270,9 +1274,6 @@ __device__ __forceinline__ void run_f32_one(const float* s, uint32_t lo, uint32_
     for (; k < hi; ++k) acc += s[k];
 }
 
-constexpr int CB = 2 * RB;           // threads of a dense chain block: bin b's g chain, then its h chain
-constexpr int CPT = WT / CB;         // positions per thread per tile
-
 // One tile of a dense chain block, CPT positions per thread, loaded a tile ahead.
 struct DenseTile {
     float g[CPT], h[CPT];
@@ -1296,7 +1297,8 @@ __device__ __forceinline__ void dense_load(DenseTile& c, const float* __restrict
     if (threadIdx.x <= NB) c.st = sf[(size_t)t * ST + threadIdx.x];
 }
 
-// Dense chains (no default bins): block (f, k), thread b (< NB) adds bin b's
+// The dense chains where features and jobs fill the CUs (chain_groups): half
+// k_tile_chain's threads and LDS, two blocks a CU.  Block (f, k), thread b (< NB) adds bin b's
 // g and thread NB + b its h, each in fp32 in row order (grow.c:55-59), from
 // the tile's pairs permuted into bucket order in LDS (channel by channel,
 // so a bin's run is contiguous); the count cell is cgrow's chain of 1.0f
@@ -1359,64 +1361,295 @@ __global__ void __launch_bounds__(CB) k_walk_chain_dense(const float* __restrict
     if (ch == 0) hist[(size_t)2 * F * NB + (size_t)f * NB + b] = (float)min(cnt, (int64_t)1 << 24);
 }
 
+// Sequential fp32 sum of the first n values at s, D sets of eight read ahead
+// of the adds (the accumulator passes through the asm after a set's reads, so
+// that the adds cannot move above them); up to 8 D cells past the run are
+// read and not added.  The last sets add +0.0f past the run, which leaves the
+// sum's bits unchanged: a sum that starts at +0.0f is never -0.0f.
+template <int D>
+__device__ __forceinline__ void run_f32(const float* s, uint32_t n, float& acc) {
+    float a[D][8];
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) a[d][u] = s[8 * d + u];
+    uint32_t r = n;                  // values left, a[0][0] the first
+    for (; r >= 8 * D; r -= 8 * D, s += 8 * D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            asm volatile("" : "+v"(acc) : : "memory");
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc += a[d][u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a[d][u] = s[8 * (D + d) + u];
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        if (__any(r > 8 * d)) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc += r > 8 * d + u ? a[d][u] : 0.0f;
+        }
+    }
+}
+
+constexpr int CDEEP = 4;             // run_f32's sets for long runs
+constexpr int CPAD = 8 * CDEEP;      // cells run_f32 may read past a tile
+
+// Bin groups per feature of a k_tile_chain launch: blocks for one a CU (every
+// group's block loads the whole tile, so more groups only repeat loads).  0
+// where features and jobs alone are more than two blocks a CU: there the
+// chains are bound by the device's throughput, and k_walk_chain_dense's
+// smaller blocks take less (1M x 100, 16 jobs a round, late rounds: 30 against
+// 34 us; 300 features, 16 jobs: a 30 000-row tree 1.25 against 1.55 ms).
+constexpr int CHAIN_BLOCKS = 256;
+inline int chain_groups(int nf, int jobs) {
+    const int64_t blocks = (int64_t)nf * jobs;
+    if (blocks > 2 * CHAIN_BLOCKS) return 0;
+    return (int)min((int64_t)8, max((int64_t)1, CHAIN_BLOCKS / blocks));
+}
+
+struct __attribute__((packed, aligned(4))) F32x4 {   // four floats at any float's address, one load
+    float v[4];
+};
+struct __attribute__((packed, aligned(8))) Pair2 {   // two rows' g, h
+    float v[4];
+};
+
+// One tile's rows of a loading thread: g, h of four rows from row
+// min(q 4 CB + 4 slot, rows left - 4) of the tile for each q < CQ (the last
+// tile's past its end read its last four again).
+struct ChainRows {
+    F32x4 g[CQ], h[CQ];
+};
+// And of its lists: entries CPT slot .. CPT slot + CPT - 1, the group's range.
+struct ChainList {
+    uint4 idx;
+    uint32_t k0, k1;
+};
+static_assert(CPT * sizeof(uint16_t) == sizeof(uint4), "a thread's list entries are one load");
+
+// Dense chains (no default bins), cgrow's row-order fp32 sums (grow.c:55-59);
+// the count cell is its chain of 1.0f adds, min(count, 2^24).  Block (feature
+// and bin group, job).  Thread b < NB runs the g chain and thread NB + b the h
+// chain of bin b0 + b of the group, from the tile's pairs in bucket order in
+// LDS (channel by channel, so a bin's run is contiguous); the other CB threads
+// put tile u's pairs by row into one buffer and tile u - 1's in bucket order
+// (the group's lists only) into another while tile u - 2 is added: one
+// barrier a tile.  Only a chain is sequential: where features and jobs leave
+// CUs idle, a feature's bins are spread over several blocks (chain_groups).
+// Rows in bins from nbins[f] on, which a caller may have, are the last group's.
+// ROOT: the node is every row, its tiles bucketed once per fit (RootOrder, its
+// largest bins give the bin count); else job blockIdx.y's built child.
+// What bounds it: the dependent adds (~15 cycles a row of the longest bin, LDS
+// reads included) at few bins, the loading threads' LDS passes (~0.8 us a tile)
+// at 256.  One block per feature and 256 adding threads took 1106 us for the
+// root of 1M x 28 at 28 bins and 312 at 256 bins; now 406 and 220 (10M x 100:
+// 3.05 -> 3.06 ms), the children of that tree 1671 -> 1300 us.  Waves that each
+// gathered their own bins' g and h from L2 with no barrier took 447 us and, at
+// 10M x 100, 10.8 ms: a 4-byte gather moves a whole line.
+template <bool ROOT>
+__global__ void __launch_bounds__(2 * CB) k_tile_chain(const float* __restrict__ Gb, const float* __restrict__ Hb,
+                                                       int64_t n, const Round* __restrict__ R, int F, int fg0, int nf,
+                                                       const uint16_t* __restrict__ perm, int64_t ld_perm,
+                                                       const uint16_t* __restrict__ starts, int64_t n_tiles,
+                                                       const int32_t* __restrict__ nbins,
+                                                       const uint8_t* __restrict__ maxbin,
+                                                       float* __restrict__ hist_base, size_t hsz) {
+    __shared__ __align__(16) float2 s_gh[2][WT + 4];            // by row, from cell 4
+    __shared__ __align__(16) float s_ch[2][2][WT + CPAD];       // g, h in bucket order
+    __shared__ uint32_t s_mb;
+    const int tid = threadIdx.x % CB, ch = tid / NB, b = tid % NB;
+    const bool adds = threadIdx.x < CB;
+    const int fl = blockIdx.x % nf, grp = blockIdx.x / nf, groups = gridDim.x / nf;
+    const int f = fg0 + fl;                        // buffers by group position, cells by feature
+    int64_t m = n, tile0 = 0;
+    const float *G = Gb, *H = Hb;
+    float* hist = hist_base;
+    if (!ROOT) {
+        const Job& J = R->job[blockIdx.y];
+        m = J.ce - J.cs;
+        tile0 = R->toff[blockIdx.y];
+        G += J.cs;
+        H += J.cs;
+        hist += (size_t)(J.build_left ? J.slot_l : J.slot_r) * hsz;
+    }
+    const int64_t tiles = (m + WT - 1) / WT;
+    const uint16_t* pf = perm + (size_t)fl * (size_t)ld_perm + (size_t)tile0 * WT;
+    const uint16_t* sf = starts + ((size_t)fl * (size_t)n_tiles + (size_t)tile0) * ST;
+    // the group's bins [b0, b0 + w)
+    int nb = NB;
+    if (groups > 1) {
+        if (ROOT) {
+            if (threadIdx.x == 0) s_mb = 0;
+            __syncthreads();
+            uint32_t mb = 0;
+            for (int64_t t = threadIdx.x; t < tiles; t += 2 * CB)
+                mb = max(mb, (uint32_t)maxbin[(size_t)f * (size_t)n_tiles + t]);
+            atomicMax(&s_mb, mb);
+            __syncthreads();
+            nb = (int)s_mb + 1;
+        } else {
+            nb = min(max(nbins[f], 1), NB);
+        }
+    }
+    const int gb = (nb + groups - 1) / groups, b0 = grp * gb;
+    if (b0 >= nb) return;
+    const int w = b0 + gb >= nb ? NB - b0 : gb;
+    float acc = 0.0f;
+    int64_t cnt = 0;
+    if (m < 4) {                                   // too few rows for the tiles' loads
+        if (adds && b < w && m > 0) {
+            const uint32_t lo = sf[b0 + b], hi = sf[b0 + b + 1];
+            for (uint32_t k = lo; k < hi; ++k) acc += (ch ? H : G)[pf[k]];
+            cnt = hi - lo;
+        }
+    } else if (adds) {
+        const uint16_t* sb = sf + b0 + min(b, w - 1);
+        uint32_t lo[2], hi[2];
+        auto bounds = [&](int k, int64_t t) {
+            const size_t at = (size_t)min(t, tiles - 1) * ST;
+            lo[k] = sb[at];
+            hi[k] = sb[at + 1];
+        };
+        bounds(0, 0);
+        bounds(1, 1);
+        __syncthreads();                           // steps 0 and 1 of the loading threads
+        __syncthreads();
+        for (int64_t u = 2; u < tiles + 2; u += 2) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int64_t t = u - 2 + k;
+                const uint32_t at = lo[k], len = t < tiles && b < w ? hi[k] - lo[k] : 0u;
+                bounds(k, t + 2);
+                if (__any(len > 64u))
+                    run_f32<CDEEP>(s_ch[k][ch] + at, len, acc);
+                else if (__any(len > 0u))
+                    run_f32<2>(s_ch[k][ch] + at, len, acc);
+                cnt += len;
+                __syncthreads();
+            }
+        }
+    } else {
+        // loads of two tiles in flight, rows a step ahead of the lists (each slot
+        // is used where it is reloaded: a copy of it would wait for its loads)
+        ChainRows rows[2];
+        ChainList list[2];
+        auto row_at = [&](int q, int64_t x0) { return min(q * 4 * CB + 4 * tid, (int)min((int64_t)WT, m - 4 - x0)); };
+        auto load_rows = [&](ChainRows& c, int64_t t) {
+            const int64_t x0 = min(t, tiles - 1) * WT;
+            const float *g = G + x0, *h = H + x0;
+#pragma unroll
+            for (int q = 0; q < CQ; ++q) c.g[q] = *reinterpret_cast<const F32x4*>(g + row_at(q, x0));
+#pragma unroll
+            for (int q = 0; q < CQ; ++q) c.h[q] = *reinterpret_cast<const F32x4*>(h + row_at(q, x0));
+        };
+        auto load_list = [&](ChainList& c, int64_t t) {
+            t = min(t, tiles - 1);
+            c.idx = *reinterpret_cast<const uint4*>(pf + t * WT + CPT * tid);   // entries past the rows: anything
+            c.k0 = sf[(size_t)t * ST + b0];
+            c.k1 = sf[(size_t)t * ST + b0 + w];
+        };
+        load_rows(rows[0], 0);
+        load_rows(rows[1], 1);
+        load_list(list[0], 0);
+        list[1].idx = make_uint4(0, 0, 0, 0);
+        list[1].k0 = list[1].k1 = 0;
+        // steps past the last tile repeat it, into cells that nothing reads
+        const int64_t steps = (tiles + 1) / 2 * 2 + 2;
+        for (int64_t u = 0; u < steps; u += 2) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                // tile u + k - 1 into bucket order: whole sets of CPT entries, so
+                // other groups' next to its own too, which nothing reads
+                const uint32_t at = CPT * tid;
+                ChainList& l = list[k ^ 1];
+                if (at + CPT > l.k0 && at < l.k1) {
+                    const uint32_t iw[4] = {l.idx.x, l.idx.y, l.idx.z, l.idx.w};
+                    float2 v[CPT];
+#pragma unroll
+                    for (int j = 0; j < CPT; ++j) v[j] = s_gh[k ^ 1][4 + ((iw[j / 2] >> (16 * (j & 1))) & (WT - 1))];
+#pragma unroll
+                    for (int j = 0; j < CPT; j += 4) {
+                        *reinterpret_cast<float4*>(&s_ch[k ^ 1][0][at + j]) =
+                            make_float4(v[j].x, v[j + 1].x, v[j + 2].x, v[j + 3].x);
+                        *reinterpret_cast<float4*>(&s_ch[k ^ 1][1][at + j]) =
+                            make_float4(v[j].y, v[j + 1].y, v[j + 2].y, v[j + 3].y);
+                    }
+                }
+                load_list(l, u + k + 1);
+                // tile u + k by row
+                ChainRows& c = rows[k];
+                const int64_t x0 = min(u + k, tiles - 1) * WT;
+#pragma unroll
+                for (int q = 0; q < CQ; ++q) {
+                    const int p = 4 + row_at(q, x0);
+                    *reinterpret_cast<Pair2*>(&s_gh[k][p]) = Pair2{{c.g[q].v[0], c.h[q].v[0], c.g[q].v[1], c.h[q].v[1]}};
+                    *reinterpret_cast<Pair2*>(&s_gh[k][p + 2]) =
+                        Pair2{{c.g[q].v[2], c.h[q].v[2], c.g[q].v[3], c.h[q].v[3]}};
+                }
+                load_rows(c, u + k + 2);
+                __syncthreads();
+            }
+        }
+    }
+    if (adds && b < w) {
+        hist[(size_t)ch * F * NB + (size_t)f * NB + b0 + b] = acc;
+        if (ch == 0) hist[(size_t)2 * F * NB + (size_t)f * NB + b0 + b] = (float)min(cnt, (int64_t)1 << 24);
+    }
+}
+
 // ---------------------------------------------------------------------------
-// the root's histogram from a per-fit rank table
+// the root's buckets, once per fit
 // ---------------------------------------------------------------------------
 //
 // The root's rows are 0 .. n - 1 in order (grow.c:289) and a fit's bins do
 // not change between its trees, so the bucketing of every (feature, WT-row
-// tile) of the root is the same for each tree of a fit.  k_root_rank computes
-// it once: for each position its rank inside its bin's run in its tile (runs
-// in row order, as k_walk_sort's), and each tile's run starts.  Each tree's
-// root then runs only the chains, k_rank_chain: one block per feature, thread
-// b = bin b, the tiles in order; a tile's g, h go into an LDS table T[rank][bin]
-// (a window of ranks at a time: RW of 256 bins, more of fewer), so that step r
-// of every thread reads its run's r-th entry from one row of T -- consecutive
-// cells across a wave, no bank conflicts -- and adds it in fp32 as cgrow does
-// (grow.c:55-59).
+// tile) of the root is the same for each tree of a fit.  k_root_order computes
+// it once, as k_walk_sort does for a child; each tree's root then runs only
+// the chains.
 
-constexpr int RW = 32;             // ranks per window of k_rank_chain's LDS table at 256 bins
-
-// The rank table of yabt_ref_root_order: ranks (uint16, F x ld_rank, position
-// t * WT + x of feature f at f * ld_rank + t * WT + x), the run starts
-// (uint16, F x tiles x ST, as k_walk_sort's), each (feature, tile)'s longest
-// run (uint16, F x tiles) and its largest bin present (uint8, F x tiles).
+// The root table of yabt_ref_root_order: each tile's positions bucketed by bin
+// (uint16, F x ld_perm), the run starts (uint16, F x tiles x ST, as
+// k_walk_sort's), each (feature, tile)'s longest run (uint16, F x tiles) and
+// its largest bin present (uint8, F x tiles).
 struct RootOrder {
-    uint16_t* rank;
+    uint16_t* perm;
     uint16_t* starts;
     uint16_t* maxrun;
     uint8_t* maxbin;
-    int64_t ld_rank;
+    int64_t ld_perm;
     int64_t tiles;
 };
 
 __host__ __device__ inline size_t root_order_carve(char* base, int64_t n, int F, RootOrder* o) {
     const int64_t tiles = (n + WT - 1) / WT > 0 ? (n + WT - 1) / WT : 1;
     const int64_t ld = tiles * WT;
-    const size_t rank_bytes = ((size_t)F * (size_t)ld * sizeof(uint16_t) + 255) / 256 * 256;
+    const size_t perm_bytes = ((size_t)F * (size_t)ld * sizeof(uint16_t) + 255) / 256 * 256;
     const size_t st_bytes = ((size_t)F * (size_t)tiles * ST * sizeof(uint16_t) + 255) / 256 * 256;
     const size_t mx_bytes = ((size_t)F * (size_t)tiles * sizeof(uint16_t) + 255) / 256 * 256;
     const size_t mb_bytes = ((size_t)F * (size_t)tiles + 255) / 256 * 256;
     if (o) {
-        o->rank = (uint16_t*)base;
-        o->starts = (uint16_t*)(base + rank_bytes);
-        o->maxrun = (uint16_t*)(base + rank_bytes + st_bytes);
-        o->maxbin = (uint8_t*)(base + rank_bytes + st_bytes + mx_bytes);
-        o->ld_rank = ld;
+        o->perm = (uint16_t*)base;
+        o->starts = (uint16_t*)(base + perm_bytes);
+        o->maxrun = (uint16_t*)(base + perm_bytes + st_bytes);
+        o->maxbin = (uint8_t*)(base + perm_bytes + st_bytes + mx_bytes);
+        o->ld_perm = ld;
         o->tiles = tiles;
     }
-    return rank_bytes + st_bytes + mx_bytes + mb_bytes;
+    return perm_bytes + st_bytes + mx_bytes + mb_bytes;
 }
 
-// Block (f, t): the ranks and run starts of feature f's tile t (tiles grid-
-// strided over y), bucketed as in k_walk_sort.
-__global__ void __launch_bounds__(RB, 8) k_root_rank(const uint8_t* __restrict__ bins_fm, int64_t ld_fm, int64_t n,
+// Block (f, t): feature f's tile t bucketed as in k_walk_sort (tiles grid-
+// strided over y).
+__global__ void __launch_bounds__(RB, 8) k_root_order(const uint8_t* __restrict__ bins_fm, int64_t ld_fm, int64_t n,
                                                   RootOrder o) {
     __shared__ uint8_t s_bin[WT];
-    __shared__ uint64_t s_peer[SW][NB];
+    __shared__ uint64_t s_peer[SW][NB];            // once the tile is ranked: its bucketed positions
     __shared__ uint32_t s_cnt[SW][NB];
     __shared__ uint32_t s_scan[SW];
     __shared__ uint32_t s_max, s_mb;
+    uint16_t* s_perm = reinterpret_cast<uint16_t*>(&s_peer[0][0]);
     const int f = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
     for (int64_t t = blockIdx.y; t < o.tiles; t += gridDim.y) {
@@ -1476,7 +1709,7 @@ __global__ void __launch_bounds__(RB, 8) k_root_rank(const uint8_t* __restrict__
             st_out[b] = (uint16_t)st;
             if (b == NB - 1) st_out[NB] = (uint16_t)(st + tb);
             // wave u's share of bin b starts c[0] + .. + c[u - 1] into the run
-            uint32_t run = 0;
+            uint32_t run = st;
 #pragma unroll
             for (int u = 0; u < SW; ++u) {
                 s_cnt[u][b] = run;
@@ -1484,322 +1717,22 @@ __global__ void __launch_bounds__(RB, 8) k_root_rank(const uint8_t* __restrict__
             }
         }
         __syncthreads();
-        uint16_t* ro = o.rank + (size_t)f * (size_t)o.ld_rank + (size_t)t0;
 #pragma unroll
         for (int q = 0; q < SGR; ++q) {
             const int x = w * SSUB + q * WAVE + lane;
-            if (x < tn) ro[x] = (uint16_t)(s_cnt[w][pk[q] >> 24] + (pk[q] & 1023u));
+            if (x < tn) s_perm[s_cnt[w][pk[q] >> 24] + (pk[q] & 1023u)] = (uint16_t)x;
         }
+        __syncthreads();
+        uint16_t* po = o.perm + (size_t)f * (size_t)o.ld_perm + (size_t)t0;
+        for (int k = tid; k < tn; k += RB) po[k] = s_perm[k];
         __syncthreads();
     }
 }
 
-// k_rank_chain's producers: RPROD threads, each loading RQ groups of four
-// positions of a tile.  Many producers with few positions each keep several
-// tiles in flight within the registers (RING tiles ahead).
-constexpr int RPROD = 2 * RB;
-constexpr int RQ = WT / (4 * RPROD);
-constexpr int RPT = 4 * RQ;                  // positions per producer and tile
-constexpr int RING = 3;
-static_assert(RQ * 4 * RPROD == WT, "a tile in whole groups of four per producer");
-
-// One tile's positions for a producer thread of k_rank_chain, RQ groups of
-// four: entry j = 4 q + k is position t WT + q 4 RPROD + 4 slot + k, so a
-// wave's 16-byte loads of g (and of h) cover 1 KB in one piece and its loads
-// of ranks and bins 512 and 256 bytes.  The tile keeps the loaded words as
-// they are: unpacking them at load time would wait for the loads there, and
-// the loads are meant to run under earlier tiles' work.
-struct RankTile {
-    float4 g[RQ], h[RQ];
-    uint2 r[RQ];                   // ranks, 16 bits each; 0xffff: past the rows
-    uint32_t bw[RQ];               // bins, 8 bits each
-};
-
-__device__ __forceinline__ float rt_g(const RankTile& c, int j) {
-    const float4 v = c.g[j >> 2];
-    return (j & 3) == 0 ? v.x : (j & 3) == 1 ? v.y : (j & 3) == 2 ? v.z : v.w;
-}
-__device__ __forceinline__ float rt_h(const RankTile& c, int j) {
-    const float4 v = c.h[j >> 2];
-    return (j & 3) == 0 ? v.x : (j & 3) == 1 ? v.y : (j & 3) == 2 ? v.z : v.w;
-}
-__device__ __forceinline__ uint32_t rt_rank(const RankTile& c, int j) {
-    const uint32_t w = (j & 2) ? c.r[j >> 2].y : c.r[j >> 2].x;
-    return (j & 1) ? (w >> 16) : (w & 0xffffu);
-}
-__device__ __forceinline__ uint32_t rt_bin(const RankTile& c, int j) { return (c.bw[j >> 2] >> (8 * (j & 3))) & 0xffu; }
-
-// A whole tile ((t + 1) WT <= n) with 16-byte aligned g, h and bins: loads
-// only, no branch (a branch joining a second way of filling the tile would
-// make the compiler wait for these loads right here).
-__device__ __forceinline__ void rank_tile_load_vec(RankTile& c, const float* __restrict__ g,
-                                                   const float* __restrict__ h, const uint8_t* __restrict__ bn,
-                                                   const uint16_t* __restrict__ rk, int64_t t, int slot) {
-    const int64_t x0 = t * WT + 4 * (int64_t)slot;
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) c.g[q] = *reinterpret_cast<const float4*>(g + x0 + q * 4 * RPROD);
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) c.h[q] = *reinterpret_cast<const float4*>(h + x0 + q * 4 * RPROD);
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) c.r[q] = *reinterpret_cast<const uint2*>(rk + x0 + q * 4 * RPROD);
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) c.bw[q] = *reinterpret_cast<const uint32_t*>(bn + x0 + q * 4 * RPROD);
-}
-
-// Any tile, one position at a time (the last, partial tile, or unaligned data).
-__device__ __forceinline__ void rank_tile_load_any(RankTile& c, const float* __restrict__ g,
-                                                   const float* __restrict__ h, const uint8_t* __restrict__ bn,
-                                                   const uint16_t* __restrict__ rk, int64_t t, int64_t n, int slot) {
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) {
-        const int64_t x = t * WT + (int64_t)q * 4 * RPROD + 4 * (int64_t)slot;
-        float gv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, hv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        uint32_t rv[4] = {0xffffu, 0xffffu, 0xffffu, 0xffffu}, bv = 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (x + k < n) {
-                gv[k] = g[x + k];
-                hv[k] = h[x + k];
-                rv[k] = rk[x + k];
-                bv |= (uint32_t)bn[x + k] << (8 * k);
-            }
-        }
-        c.g[q] = make_float4(gv[0], gv[1], gv[2], gv[3]);
-        c.h[q] = make_float4(hv[0], hv[1], hv[2], hv[3]);
-        c.r[q] = make_uint2(rv[0] | (rv[1] << 16), rv[2] | (rv[3] << 16));
-        c.bw[q] = bv;
-    }
-}
-
-// One window of a tile's entries, g and h in separate tables: a producer
-// writes each value as it was loaded (pairing g with h for one 8-byte store
-// would have the compiler permute the loaded registers right after the
-// loads, which waits for them).  Cell (r, b) is at (r << lg) + b, where
-// 2^lg >= 1 + the feature's largest bin: a window holds RW NB >> lg ranks, so
-// a feature of few bins (long runs per tile) takes a tile in one window.
-struct RankTable {
-    float g[RW * NB];
-    float h[RW * NB];
-};
-
-// A producer's window [w0, w0 + rw) of its tile's entries into T[rank - w0][bin]
-// (rw = RW NB >> lg; a bin past 2^lg, which the rank table rules out, is
-// dropped rather than written into another rank's cells).
-__device__ __forceinline__ void rank_stage(const RankTile& c, RankTable& T, uint32_t w0, uint32_t rw, int lg) {
-#pragma unroll
-    for (int j = 0; j < RPT; ++j) {
-        // a rank below w0 wraps above rw; past the rows the rank is 0xffff
-        const uint32_t rank = rt_rank(c, j), r = rank - w0;
-        const uint32_t b = rt_bin(c, j);
-        if (rank != 0xffffu && r < rw && (b >> lg) == 0) {
-            T.g[(r << lg) + b] = rt_g(c, j);
-            T.h[(r << lg) + b] = rt_h(c, j);
-        }
-    }
-}
-
-// Block f: the root's fp32 cells of feature f, cgrow's row-order chains
-// (grow.c:37-62); the count cell is cgrow's chain of 1.0f adds,
-// min(count, 2^24).  Threads 0 .. RB - 1 are the consumers, thread b adding
-// bin b's run of each tile in rank order from an LDS table T[rank][bin]
-// (2^lg bins a rank, lg from the largest bin of the feature's tiles);
-// threads RB .. RB + RPROD - 1 are the producers, filling the other of two
-// tables with the next tile meanwhile (window 0 of every tile; a tile whose
-// longest run passes the window has its further windows staged and added in turn,
-// its positions reloaded).  The producers' next tiles load RING tiles ahead:
-// a step is shorter than a load's latency under load.  VEC:
-// g, h and the bins are 16-byte aligned (every feature's column:
-// ld_fm % 16 == 0).
-template <bool VEC>
-__global__ void __launch_bounds__(RB + RPROD) k_rank_chain(const float* __restrict__ g, const float* __restrict__ h,
-                                                       const uint8_t* __restrict__ bins_fm, int64_t ld_fm, int64_t n,
-                                                       RootOrder o, float* __restrict__ hist, int F) {
-    __shared__ RankTable T[2];
-    __shared__ uint32_t s_mb;
-    const int f = blockIdx.x;
-    const bool prod = threadIdx.x >= RB;
-    const int lt = prod ? (int)threadIdx.x - RB : (int)threadIdx.x;   // consumers: the bin; producers: the slot
-    const uint8_t* bn = bins_fm + (size_t)f * (size_t)ld_fm;
-    const uint16_t* rk = o.rank + (size_t)f * (size_t)o.ld_rank;
-    const uint16_t* sf = o.starts + (size_t)f * (size_t)o.tiles * ST;
-    const uint16_t* mx = o.maxrun + (size_t)f * (size_t)o.tiles;
-    const int64_t tiles = (n + WT - 1) / WT;
-    const int64_t full = VEC ? n / WT : 0;      // tiles the producers load with 16-byte loads
-    {
-        if (threadIdx.x == 0) s_mb = 0;
-        __syncthreads();
-        uint32_t m = 0;
-        const uint8_t* mb = o.maxbin + (size_t)f * (size_t)o.tiles;
-        for (int64_t t = threadIdx.x; t < tiles; t += blockDim.x) m = max(m, (uint32_t)mb[t]);
-        atomicMax(&s_mb, m);
-        __syncthreads();
-    }
-    const int lg = 32 - __builtin_clz(__builtin_amdgcn_readfirstlane((int)s_mb) | 1);   // 2^lg > the largest bin
-    const uint32_t rw = (uint32_t)(RW * NB) >> lg;                                     // ranks per window
-    // consumers: at 256 bins (both) thread lt runs both chains of bin lt;
-    // below, thread lt runs the one chain of channel cch = lt >> lg (0: g,
-    // 1: h) of bin cb = lt mod 2^lg, and threads from 2^(lg + 1) on idle
-    const bool both = lg == 8;
-    const int cb = both ? lt : (lt & ((1 << lg) - 1));
-    const int cch = both ? 0 : (lt >> lg);
-    const bool live = prod || cch < 2;
-    float ag = 0.0f, ah = 0.0f;   // both: g and h; else: channel cch in ag
-    int64_t cnt = 0;
-    // consumer: window [w0, w0 + rw) of tile t's run of its bin from table Tb;
-    // steps to the tile's longest run in the window (uniform); past this
-    // thread's run a step adds +0.0f, which leaves the sums' bits unchanged (a
-    // sum that starts at +0.0f is never -0.0f).  Both chains: eight ranks'
-    // reads in flight, then their adds.
-    auto run2 = [&](const RankTable& Tb, uint32_t len, uint32_t mr, uint32_t w0) {
-        const uint32_t kend = min(len > w0 ? len - w0 : 0u, rw);
-        const uint32_t kmax = min(mr - w0, rw);
-        for (uint32_t r = 0; r < kmax; r += 8) {
-            float vg[8], vh[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                vg[u] = Tb.g[((r + u) << 8) + lt];
-                vh[u] = Tb.h[((r + u) << 8) + lt];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const bool in = r + u < kend;
-                ag += in ? vg[u] : 0.0f;
-                ah += in ? vh[u] : 0.0f;
-            }
-        }
-    };
-    // One chain (tb: the channel's table at the bin's column), sixteen ranks a
-    // turn in two register sets: each set's next reads are issued before the
-    // other set's adds (the accumulator passes through the asm after the
-    // reads, so the adds cannot move above them); groups past the window
-    // read a clamped group in it, unused.
-    auto run1 = [&](const float* tb, uint32_t len, uint32_t mr, uint32_t w0) {
-        const uint32_t kend = min(len > w0 ? len - w0 : 0u, rw);
-        const uint32_t kmax = min(mr - w0, rw);
-        if (kmax == 0) return;
-        float a[8], b[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) a[u] = tb[u << lg];
-        for (uint32_t r = 0; r < kmax; r += 16) {
-            const uint32_t rb = min(r + 8, rw - 8), ra = min(r + 16, rw - 8);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) b[u] = tb[(rb + u) << lg];
-            asm volatile("" : "+v"(ag) : : "memory");
-#pragma unroll
-            for (int u = 0; u < 8; ++u) ag += r + u < kend ? a[u] : 0.0f;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) a[u] = tb[(ra + u) << lg];
-            asm volatile("" : "+v"(ag) : : "memory");
-#pragma unroll
-            for (int u = 0; u < 8; ++u) ag += r + 8 + u < kend ? b[u] : 0.0f;
-        }
-    };
-    auto run = [&](const RankTable& Tb, uint32_t len, uint32_t mr, uint32_t w0) {
-        if (both)
-            run2(Tb, len, mr, w0);
-        else
-            run1((cch ? Tb.h : Tb.g) + cb, len, mr, w0);
-    };
-    auto load = [&](RankTile& c, int64_t t) {
-        if (t < full)
-            rank_tile_load_vec(c, g, h, bn, rk, t, lt);
-        else
-            rank_tile_load_any(c, g, h, bn, rk, t, n, lt);
-    };
-    // every thread: tile t's longest run, RING tiles ahead in mrs[t % RING];
-    // consumers: their bin's run start and end in the tile, in se[t % RING]
-    // (a load used in the step it is issued would put a memory latency on
-    // every tile's path)
-    uint32_t mrs[RING], se[RING];
-    const uint16_t* sfl = sf + (prod ? 0 : cb);   // consumers' start entries: tile t at sfl[t ST], its end at sfl[t ST + 1]
-    auto meta = [&](int k, int64_t t) {
-        if (t < tiles) {
-            mrs[k] = mx[t];
-            if (!prod) se[k] = (uint32_t)sfl[(size_t)t * ST] | ((uint32_t)sfl[(size_t)t * ST + 1] << 16);
-        }
-    };
-#pragma unroll
-    for (int k = 0; k < RING; ++k) meta(k, k);
-    // producers: tile 0's window 0, and the ring (tiles 1 .. RING)
-    RankTile ring[RING];
-    if (prod && tiles > 0) {
-        RankTile c;
-        load(c, 0);
-        rank_stage(c, T[0], 0, rw, lg);
-    }
-    if (prod && full > 0) {
-#pragma unroll
-        for (int k = 0; k < RING; ++k) rank_tile_load_vec(ring[k], g, h, bn, rk, min((int64_t)(1 + k), full - 1), lt);
-    }
-    __syncthreads();
-    // step t: the consumers add tile t's window 0 from T[t & 1] while the
-    // producers stage tile t + 1's from ring slot R (then reload R with tile
-    // t + 1 + RING); then tile t's further windows, if any
-    auto step = [&](int64_t t, RankTile& R, int k) {
-        if (t >= tiles) return;
-        const uint32_t mr = (uint32_t)__builtin_amdgcn_readfirstlane((int)mrs[k]);
-        uint32_t len = 0;
-        if (!prod) len = (se[k] >> 16) - (se[k] & 0xffffu);
-        meta(k, t + RING);
-        if (!prod) {
-            if (live) run(T[t & 1], len, mr, 0);
-            cnt += len;
-        } else if (t + 1 < tiles) {
-            if (t + 1 < full) {
-                rank_stage(R, T[(t + 1) & 1], 0, rw, lg);
-            } else {
-                RankTile c;
-                rank_tile_load_any(c, g, h, bn, rk, t + 1, n, lt);
-                rank_stage(c, T[(t + 1) & 1], 0, rw, lg);
-            }
-        }
-        if (prod && full > 0) rank_tile_load_vec(R, g, h, bn, rk, min(t + 1 + RING, full - 1), lt);
-        __syncthreads();
-        for (uint32_t w0 = rw; w0 < mr; w0 += rw) {
-            if (prod) {
-                RankTile c;
-                load(c, t);
-                rank_stage(c, T[t & 1], w0, rw, lg);
-            }
-            __syncthreads();
-            if (!prod && live) run(T[t & 1], len, mr, w0);
-            __syncthreads();
-        }
-    };
-    for (int64_t t = 0; t < tiles; t += RING) {
-#pragma unroll
-        for (int k = 0; k < RING; ++k) step(t + k, ring[k], k);
-    }
-    // below 256 bins the chains' sums meet in LDS (T[0], free after the last
-    // step's barrier): s_o[ch NB + bin], the counts at T[0].h; bins from 2^lg
-    // on are empty
-    float* s_o = T[0].g;
-    __syncthreads();
-    if (!both && !prod && cch < 2) s_o[cch * NB + cb] = ag;
-    if (!both && !prod && cch == 0) T[0].h[cb] = (float)min(cnt, (int64_t)1 << 24);
-    __syncthreads();
-    if (!prod) {
-        float vg = ag, vh = ah, vc = (float)min(cnt, (int64_t)1 << 24);
-        if (!both) {
-            const bool in = (lt >> lg) == 0;
-            vg = in ? s_o[lt] : 0.0f;
-            vh = in ? s_o[NB + lt] : 0.0f;
-            vc = in ? T[0].h[lt] : 0.0f;
-        }
-        hist[(size_t)f * NB + lt] = vg;
-        hist[(size_t)F * NB + (size_t)f * NB + lt] = vh;
-        hist[(size_t)2 * F * NB + (size_t)f * NB + lt] = vc;
-    }
-}
-
-inline void launch_rank_chain(const float* g, const float* h, const uint8_t* bins_fm, int64_t ld_fm, int64_t n,
-                              const RootOrder& o, float* hist, int F, hipStream_t stream) {
-    const bool vec = ((uintptr_t)g % 16 == 0) && ((uintptr_t)h % 16 == 0) && ((uintptr_t)bins_fm % 16 == 0) &&
-                     (ld_fm % 16 == 0);
-    if (vec)
-        k_rank_chain<true><<<F, RB + RPROD, 0, stream>>>(g, h, bins_fm, ld_fm, n, o, hist, F);
-    else
-        k_rank_chain<false><<<F, RB + RPROD, 0, stream>>>(g, h, bins_fm, ld_fm, n, o, hist, F);
+inline void launch_root_chain(const float* g, const float* h, int64_t n, const RootOrder& o, float* hist, int F,
+                              hipStream_t stream) {
+    k_tile_chain<true><<<(unsigned)(F * max(1, chain_groups(F, 1))), 2 * CB, 0, stream>>>(
+        g, h, n, nullptr, F, 0, F, o.perm, o.ld_perm, o.starts, o.tiles, nullptr, o.maxbin, hist, 0);
 }
 
 // Sparse builder's default-bin cells (grow.c:101-106): 0 + (float)(node sum -
@@ -2167,6 +2100,7 @@ struct Grower {
     Ws w;
     size_t hsz;
     const int32_t* dbin;           // sparse builder's default bins, or null
+    const int32_t* nbins;          // bins per feature
     hipStream_t st;
 
     // Histograms of the round's K built children (the root: every row), in
@@ -2197,6 +2131,9 @@ struct Grower {
             if (dbin)
                 k_walk_chain_sparse<<<cgrid, RB, 0, st>>>(G, H, w.round, F, fg0, nf, dbin, w.perm, w.xperm, w.ld_perm,
                                                           w.starts, w.n_tiles, w.hist, hsz, w.tries, w.expl, w.tot);
+            else if (chain_groups(nf, K) > 0)
+                k_tile_chain<false><<<dim3((unsigned)(nf * chain_groups(nf, K)), (unsigned)K), 2 * CB, 0, st>>>(
+                    G, H, n, w.round, F, fg0, nf, w.perm, w.ld_perm, w.starts, w.n_tiles, nbins, nullptr, w.hist, hsz);
             else
                 k_walk_chain_dense<<<cgrid, CB, 0, st>>>(G, H, w.round, F, fg0, w.perm, w.ld_perm, w.starts,
                                                          w.n_tiles, w.hist, hsz);
@@ -2250,7 +2187,7 @@ int yabt_ref_root_order(const uint8_t* bins_fm, int64_t ld_fm, int64_t n, int F,
     RootOrder o;
     root_order_carve((char*)out, n, F, &o);
     const unsigned ty = (unsigned)min((int64_t)65535, o.tiles);
-    k_root_rank<<<dim3((unsigned)F, ty), RB, 0, stream>>>(bins_fm, ld_fm, n, o);
+    k_root_order<<<dim3((unsigned)F, ty), RB, 0, stream>>>(bins_fm, ld_fm, n, o);
     return launch_status("yabt_ref_root_order launch");
 }
 
@@ -2263,7 +2200,7 @@ int yabt_ref_root_hist(const uint8_t* bins_fm, int64_t ld_fm, const float* grad,
         return fail(-2, "yabt_ref_root_hist: root_order smaller than yabt_ref_root_order_bytes(n, F)");
     RootOrder o;
     root_order_carve((char*)const_cast<void*>(root_order), n, F, &o);
-    launch_rank_chain(grad, hess, bins_fm, ld_fm, n, o, out, F, stream);
+    launch_root_chain(grad, hess, n, o, out, F, stream);
     return launch_status("yabt_ref_root_hist launch");
 }
 
@@ -2315,6 +2252,7 @@ int yabt_grow_ref(const uint8_t* bins_fm, int64_t ld_fm, const uint8_t* bins_rm,
     g.w = carve((char*)workspace, n, F, max_leaves, sparse, fgroup);
     g.hsz = (size_t)3 * F * NB;
     g.dbin = default_bin;
+    g.nbins = nbins;
     g.st = stream;
     const Ws& w = g.w;
     const int N = 2 * max_leaves + 1;
@@ -2411,7 +2349,7 @@ int yabt_grow_ref(const uint8_t* bins_fm, int64_t ld_fm, const uint8_t* bins_rm,
         if (root_order && !sparse && n > 0) {
             RootOrder o;
             root_order_carve((char*)const_cast<void*>(root_order), n, F, &o);
-            launch_rank_chain(grad, hess, bins_fm, ld_fm, n, o, w.hist, F, stream);
+            launch_root_chain(grad, hess, n, o, w.hist, F, stream);
         } else {
             g.hist(true, 1, R.toff[1], grad, hess);
         }

@@ -136,11 +136,11 @@ class BinLayouts:
         return self._counts
 
     def ref_root_order(self) -> torch.Tensor:
-        """The root rank table of the reference-arithmetic grower's dense
-        builder (yabt_ref_root_order), built once per layout: each row's rank
-        in its bin inside its 4096-row tile, per feature, which every tree's
+        """The root table of the reference-arithmetic grower's dense
+        builder (yabt_ref_root_order), built once per layout: each 4096-row
+        tile's rows bucketed by bin, per feature, which every tree's
         root histogram on these bins reuses.  F * ceil(n / 4096) * 4096
-        uint16 ranks plus the tiles' bin starts (yabt_ref_root_order_bytes):
+        uint16 positions plus the tiles' bin starts (yabt_ref_root_order_bytes):
         2.0 GB at 10M rows x 100 features, kept until the layout dies or
         release_ref_root_order() drops it."""
         if self._root_order is None:
@@ -158,7 +158,7 @@ class BinLayouts:
         return self._root_order
 
     def release_ref_root_order(self) -> None:
-        """Drop the reference-arithmetic root rank table (the largest per-fit
+        """Drop the reference-arithmetic root table (the largest per-fit
         table, see ref_root_order); the next reference-arithmetic tree on this
         layout rebuilds it.  Call it when no grower on this layout is running:
         the memory goes back to torch's caching allocator (the device is
@@ -475,7 +475,7 @@ def _grow_device_ref(lay: BinLayouts, grad, hess, nbins, *, fmask, imat, ib, lam
     library's recommended size) may be anything from
     yabt_grow_ref_workspace_min_bytes up: features are bucketed in groups
     that fit.  root_order: the dense builder's root reads the layout's cached
-    rank table (BinLayouts.ref_root_order) instead of bucketing every tree."""
+    root table (BinLayouts.ref_root_order) instead of bucketing every tree."""
     lib = _lib.load()
     dev = lay.fm.device
     n, F = lay.n, lay.F
@@ -660,7 +660,7 @@ def hist(lay: BinLayouts, grad: torch.Tensor, hess: torch.Tensor,
 def ref_root_hist(lay: BinLayouts, grad: torch.Tensor, hess: torch.Tensor) -> torch.Tensor:
     """The root's (3, F, 256) float32 histogram in the reference arithmetic
     (cgrow's row-order fp32 sums, grow.c:37-62), from the layout's cached
-    root rank table."""
+    root table."""
     lib = _lib.load()
     dev = lay.fm.device
     g = _dev_f32(grad, dev)
