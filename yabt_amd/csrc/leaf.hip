@@ -1115,11 +1115,19 @@ __global__ void __launch_bounds__(LB) k_leaf_fold(int n_nodes, int K, const floa
 // order (per-block partials, then one block), so the result is deterministic
 // ---------------------------------------------------------------------------
 
-constexpr int MROWS = 16384;                   // rows per moments block
+// Rows per moments block, a function of n alone (the partials' order is the
+// result's): about 512 blocks, since a thread waits for its rows' loads one
+// group after the other (16384 rows a block: 41 us at 2M rows, 34 at 20 000;
+// now 18 and 7).
+constexpr int64_t MROWS_MIN = 1024, MROWS_MAX = 16384, MBLOCKS = 512;
+inline int64_t moment_rows(int64_t n) {
+    const int64_t per = ((n + MBLOCKS - 1) / MBLOCKS + LB - 1) / LB * LB;
+    return per < MROWS_MIN ? MROWS_MIN : per > MROWS_MAX ? MROWS_MAX : per;
+}
 
 // fp32 inputs: per-block fp64 partials of x and x^2.
 template <int K>
-__global__ void __launch_bounds__(LB) k_leaf_moments(int x_kind, const void* X, int64_t ldx, int64_t n,
+__global__ void __launch_bounds__(LB) k_leaf_moments(int x_kind, const void* X, int64_t ldx, int64_t n, int64_t rows,
                                                      const int32_t* feats, double* part) {
     __shared__ int32_t s_fs[LKMAX];
     __shared__ double s_red[LB / WAVE][2 * LKMAX];
@@ -1129,7 +1137,7 @@ __global__ void __launch_bounds__(LB) k_leaf_moments(int x_kind, const void* X, 
     A.x_kind = x_kind;
     A.X = X;
     A.ldx = ldx;
-    const int64_t lo = (int64_t)blockIdx.x * MROWS, hi = min(n, lo + MROWS);
+    const int64_t lo = (int64_t)blockIdx.x * rows, hi = min(n, lo + rows);
     double s1[K], s2[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) s1[j] = s2[j] = 0.0;
@@ -1297,20 +1305,21 @@ int64_t gram_slots(Kern kern, size_t lds) {
     return slots;
 }
 
-// GRAM_ACC's chunk: LCHUNK positions, or, when that makes more than one full
-// wave of resident blocks, the size that makes the chunk count a whole
-// multiple of them (a last, partial wave of blocks had left most of the
-// device idle for a block's lifetime: 2442 chunks of 4096 at 10M rows on
-// 1024 slots), rounded up to whole rows per thread and kept at most
-// (LB / 2) 2^(k - 11) so that a thread adds at most 2^(k - 11) products per
-// entry and segment (k = ceil(log2 n) >= 16 here).
+// The exact Gram's chunk: about LCHUNK positions where that fills the resident
+// blocks, sized so that the chunk count is a whole multiple of them (a last,
+// partial wave of blocks had left most of the device idle for a block's
+// lifetime: 2442 chunks of 4096 at 10M rows on 1024 slots); of fewer rows one
+// chunk per resident block, down to GRAM_MIN positions (20 000 rows: 35 us in 5
+// chunks of 4096, 10 in 79).  Whole
+// rows per thread; for GRAM_ACC (above 32768 rows) at most (LB / 2) 2^(k - 11),
+// so that a thread adds at most 2^(k - 11) products per entry and segment
+// (k = ceil(log2 n) >= 16 here).
+constexpr int64_t GRAM_MIN = 256;
 inline int64_t gram_chunk(int64_t n, int64_t slots) {
-    int64_t chunk = LCHUNK;
-    const int64_t waves = n / (slots * LCHUNK);
-    if (waves >= 1) {
-        chunk = (n + slots * waves - 1) / (slots * waves);
-        chunk = (chunk + LB / 2 - 1) / (LB / 2) * (LB / 2);
-    }
+    const int64_t waves = std::max<int64_t>(1, n / (slots * LCHUNK));
+    int64_t chunk = std::max<int64_t>(GRAM_MIN, (n + slots * waves - 1) / (slots * waves));
+    chunk = (chunk + LB / 2 - 1) / (LB / 2) * (LB / 2);
+    if (n <= 32768) return chunk;
     int k = 0;
     while (k < 62 && ((int64_t)1 << k) < n) ++k;
     const int64_t cap = (int64_t)(LB / 2) << (k > 11 ? k - 11 : 0);
@@ -1347,8 +1356,7 @@ void launch_leaf_fit(LeafArgs& A, float* out_W, float* out_b, float* out_lo, flo
             k_leaf_reduce<K><<<A.n_nodes, RB, 0, stream>>>(A);
         } else {
             // dynamic LDS: the chunk's segment list
-            A.gram_chunk = LCHUNK;
-            if (A.n > 32768) A.gram_chunk = gram_chunk(A.n, gram_slots(k_leaf_gram<K, GRAM_ACC>, 0));
+            A.gram_chunk = gram_chunk(A.n, gram_slots(k_leaf_gram<K, GRAM_ACC>, 0));
             const size_t seg_lds = sizeof(int) * (size_t)std::min<int64_t>(A.n_nodes, A.gram_chunk);
             const int gc = (int)((A.n + A.gram_chunk - 1) / A.gram_chunk);
             if (A.n > 32768) k_leaf_gram<K, GRAM_ACC><<<gc, LB, seg_lds, stream>>>(A);
@@ -1692,7 +1700,7 @@ int yabt_leaf_rank_features(const int64_t* feature, int n_nodes, int F, int k, i
 
 size_t yabt_leaf_moments_workspace_bytes(int64_t n) {
     if (n < 0) return 0;
-    const int64_t nb = n > 0 ? (n + MROWS - 1) / MROWS : 1;
+    const int64_t mr = moment_rows(n), nb = n > 0 ? (n + mr - 1) / mr : 1;
     const size_t f = (size_t)nb * 2 * LKMAX * sizeof(double), u = (size_t)MU8_BLOCKS * LKMAX * 2 * sizeof(uint64_t);
     return align_up(f > u ? f : u, 256);
 }
@@ -1704,7 +1712,8 @@ int yabt_leaf_moments(int x_kind, const void* X, int64_t ldx, int64_t n, const i
     if (!X || !feats || !workspace || !out_mu || !out_sd) return fail(-2, "yabt_leaf_moments: null pointer argument");
     if (x_kind != 0 ? ldx < n : ldx < 1) return fail(-2, "yabt_leaf_moments: leading dimension too small");
     if (workspace_bytes < yabt_leaf_moments_workspace_bytes(n)) return fail(-2, "yabt_leaf_moments: workspace too small");
-    const int nb = (int)((n + MROWS - 1) / MROWS);
+    const int64_t mr = moment_rows(n);
+    const int nb = (int)((n + mr - 1) / mr);
     double* part = (double*)workspace;
     if (x_kind == 1) {
         const int gb = launch_grid((n + 15) / 16, LB, MU8_BLOCKS);
@@ -1713,14 +1722,14 @@ int yabt_leaf_moments(int x_kind, const void* X, int64_t ldx, int64_t n, const i
         return launch_status("yabt_leaf_moments launch");
     }
     switch (K) {
-        case 1: k_leaf_moments<1><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, feats, part); break;
-        case 2: k_leaf_moments<2><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, feats, part); break;
-        case 3: k_leaf_moments<3><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, feats, part); break;
-        case 4: k_leaf_moments<4><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, feats, part); break;
-        case 5: k_leaf_moments<5><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, feats, part); break;
-        case 6: k_leaf_moments<6><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, feats, part); break;
-        case 7: k_leaf_moments<7><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, feats, part); break;
-        default: k_leaf_moments<8><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, feats, part); break;
+        case 1: k_leaf_moments<1><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, mr, feats, part); break;
+        case 2: k_leaf_moments<2><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, mr, feats, part); break;
+        case 3: k_leaf_moments<3><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, mr, feats, part); break;
+        case 4: k_leaf_moments<4><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, mr, feats, part); break;
+        case 5: k_leaf_moments<5><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, mr, feats, part); break;
+        case 6: k_leaf_moments<6><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, mr, feats, part); break;
+        case 7: k_leaf_moments<7><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, mr, feats, part); break;
+        default: k_leaf_moments<8><<<nb, LB, 0, stream>>>(x_kind, X, ldx, n, mr, feats, part); break;
     }
     k_leaf_moments_final<<<K, WAVE, 0, stream>>>(part, nb, n, K, out_mu, out_sd);
     return launch_status("yabt_leaf_moments launch");
