@@ -320,8 +320,8 @@ def reference_arithmetic(torch, lay, g, h, nbins, steps: int, exact_res, neural:
     """The same tree grown with the reference's own fp32 arithmetic
     (yabt_grow_ref, whose trees equal grow.c's node for node): ms per tree for
     the grower alone and with the leaf models, its root histogram (cgrow's
-    row-order fp32 chains from the per-fit rank table) with its share of HBM
-    peak, the per-fit rank table's cost, and the internal nodes whose
+    row-order fp32 chains from the per-fit root table) with its share of HBM
+    peak, the per-fit root table's cost, and the internal nodes whose
     (feature, bin) differ from the exact tree's."""
     from yabt_amd import grow_hip as G
     from yabt_amd.neural_leaves import fit_leaf_networks_binned
@@ -373,9 +373,9 @@ def reference_arithmetic(torch, lay, g, h, nbins, steps: int, exact_res, neural:
     root_bytes = n * F + 8 * n
     out["root_hist"] = {"ms": round(root_ms, 3), "GBps": round(root_bytes / (root_ms * 1e-3) / 1e9, 1),
                         "frac_hbm": round(root_bytes / (root_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                        "kernel": "k_rank_chain (row-order fp32 chains, one block per feature)"}
+                        "kernel": "k_tile_chain (row-order fp32 chains, a feature's bins over up to eight blocks)"}
     out["fit_setup"] = {"root_order_ms": round(order_ms, 2),
-                        "note": "per-fit root rank table (yabt_ref_root_order), outside the step"}
+                        "note": "per-fit root table (yabt_ref_root_order), outside the step"}
     # split sequence against the exact tree's
     a = {k: getattr(exact_res, k)[:exact_res.n_nodes].cpu().numpy() for k in ("feature", "thr_bin", "left")}
     b = {k: getattr(res, k)[:res.n_nodes].cpu().numpy() for k in ("feature", "thr_bin", "left")}
