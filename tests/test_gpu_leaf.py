@@ -122,6 +122,28 @@ def test_leaf_moments(n, K, x_kind):
     assert np.array_equal(a[0], m) and np.array_equal(a[1], s)
 
 
+@pytest.mark.parametrize("n,K,n_nodes", [(255, 2, 5), (257, 8, 7), (1024, 3, 7), (1025, 8, 7), (32_768, 8, 63),
+                                         (32_769, 5, 63), (524_288, 8, 63), (524_289, 4, 63)])
+def test_leaf_blocks_at_their_edges(n, K, n_nodes):
+    """One row around the sizes where the moments' rows per block change
+    (1024 up to 524 288 rows, whole multiples of the block above) and where the
+    exact Gram's chunk does (256 positions at few rows; the accumulating form
+    above 32 768).  Moments: fp64 sums, each side rounded once to fp32 (two half
+    ulps, 1.2e-7 relative); fits as in test_leaf_fit_matches_oracle."""
+    X, Xf, feats, g, h, feature, leaf, mu, sd = _problem(n, n, K, n_nodes)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+    m, s = (v.cpu().numpy() for v in leaf_moments(t(X), 0, t(feats), n))
+    rm, rs = NO.moments(Xf[:, feats])
+    np.testing.assert_allclose(m, rm, rtol=2e-7, atol=0)
+    np.testing.assert_allclose(s, rs, rtol=2e-7, atol=0)
+    W, b, lo, hi, cnt = _gpu(X, 0, feats, g, h, feature, leaf, mu, sd, 50, 1.0)
+    rW, rb, rlo, rhi, rcnt = _oracle(Xf, feats, g, h, feature, leaf, mu, sd, 50, 1.0)
+    assert np.array_equal(cnt, rcnt)
+    assert np.array_equal(lo, rlo) and np.array_equal(hi, rhi)
+    np.testing.assert_allclose(W, rW, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(b, rb, rtol=1e-5, atol=1e-6)
+
+
 @pytest.mark.parametrize("gram", ["exact", "mfma"])
 def test_leaf_fit_deterministic_and_u8_equals_f32(gram):
     """Exact sums: identical bits on every call and for either input path.
