@@ -380,8 +380,10 @@ size_t yabt_grow_ref_workspace_min_bytes(int64_t n, int F, int max_leaves, int s
  * bucketed in the call): the root table yabt_ref_root_order made for these
  * bins_fm, n and F, which the dense builder's root then reads instead of
  * bucketing its rows again (the sparse builder ignores it).  The call returns
- * after the stream has finished (it synchronises `stream`).  Requires
- * n < 2^32, F >= 1, 1 <= max_leaves <= 32767. */
+ * after the stream has finished (it synchronises `stream`).  bins_fm may have
+ * any address and any ld_fm >= n (16-byte aligned columns are read faster),
+ * root_order any even address.  Requires n < 2^32, F >= 1,
+ * 1 <= max_leaves <= 32767. */
 int yabt_grow_ref(const uint8_t *bins_fm, int64_t ld_fm, const uint8_t *bins_rm, int64_t ld_rm,
                   const float *grad, const float *hess, const uint8_t *fmask, const float *imat,
                   float ib, int use_imat, const int32_t *nbins, const int32_t *default_bin,

@@ -3,11 +3,16 @@ the root's histogram bit for bit against the oracle's row-order fp32 sums
 (oracle/grow_oracle.c, grow.c:37-62) at the edges of a tile, of its four-row
 loads and of the bin groups, and trees through either kernel."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
+from oracle import boost_oracle as BO
 from oracle import oracle as O
+from tests.helpers import tree_arrays_equal
+from yabt_amd import _lib
 from yabt_amd import grow_hip as G
 
 pytestmark = pytest.mark.gpu
@@ -58,3 +63,36 @@ def test_bucketed_root_and_children(n, F, top, nb):
         want = O.grow(np.ascontiguousarray(bins.T), g, h, mode=O.MODE_FP32, nbins=nbins, msl=5, max_leaves=63)
         assert np.array_equal(a.feature.cpu().numpy(), want["feature"])
         assert np.array_equal(a.value.cpu().numpy().view(np.uint32), want["value"].view(np.uint32))
+
+
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("n,offset", [(4099, 0), (8192, 1), (5003, 1)])   # the columns' length, or their start, is no multiple of 16
+def test_columns_that_no_wide_load_fits(n, offset, sparse):
+    """Feature-major columns without padding or alignment, and a root table
+    that starts two bytes into its buffer: the oracle's tree."""
+    F = 3
+    bins, g, h = _data(n, F, 200)
+    whole = G.make_layouts(torch.from_numpy(bins), DEV)
+    buf = torch.empty(offset + F * n, dtype=torch.uint8, device=DEV)
+    fm = buf[offset:].view(F, n)
+    fm.copy_(torch.from_numpy(np.ascontiguousarray(bins.T)))
+    lay = G.BinLayouts(fm, whole.rm, n, F)
+    layout = BO.sparse_layout(bins) if sparse else None
+    nbins = np.full(F, 256, np.int32)
+    kw = dict(lam=1.0, gamma=0.0, mcw=1e-3, msl=5, lr=0.1, max_leaves=15, max_depth=64)
+    want = O.grow(np.ascontiguousarray(bins.T), g, h, mode=O.MODE_FP32, nbins=nbins, sparse=layout, msl=5, max_leaves=15)
+    tables = [False] if sparse else [False, True]
+    if not sparse:
+        lib = _lib.load()
+        nb = int(lib.yabt_ref_root_order_bytes(n, F))
+        tab = torch.empty(nb + 2, dtype=torch.uint8, device=DEV)
+        _lib.check(lib.yabt_ref_root_order(ctypes.c_void_p(fm.data_ptr()), n, n, F, ctypes.c_void_p(tab.data_ptr() + 2), nb,
+                                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "yabt_ref_root_order")
+        lay._root_order = tab[2:]
+    for table in tables:
+        print(f"unpadded columns: n={n} offset={offset} sparse={sparse} table={table}", flush=True)
+        res = G._grow_device_ref(lay, torch.from_numpy(g).to(DEV), torch.from_numpy(h).to(DEV), nbins, fmask=None, imat=None,
+                                 ib=0.0, default_bin=layout[3] if sparse else None, root_order=table, **kw)
+        got = {k: getattr(res, k).cpu().numpy() for k in ("feature", "thr_bin", "left", "right", "value", "depth")}
+        assert tree_arrays_equal(got, want) is None
+        assert np.array_equal(res.rows.cpu().numpy(), want["rows"])

@@ -397,14 +397,15 @@ constexpr int TPT = WT / RB;              // rows per thread per tile
 
 // Bins of a tile's tn rows (row t0 + x of the node) into s_bin: from the
 // feature-major column for the root (rows[] is the identity there,
-// grow.c:289; t0 % 16 == 0 and the column is padded to 16 rows), 16 rows a
-// thread with one load; by row id from the row-major copy else.
+// grow.c:289; t0 % 16 == 0), 16 rows a thread with one load where every column
+// is 16-byte aligned and padded to 16 rows, else a row a load; by row id from
+// the row-major copy else.
 template <bool ROOT>
 __device__ __forceinline__ void tile_bins(const uint8_t* __restrict__ bins_fm, int64_t ld_fm,
                                           const uint8_t* __restrict__ bins_rm, int64_t ld_rm,
                                           const uint32_t* __restrict__ crow, int f, int64_t t0, int tn, uint8_t* s_bin) {
     const int tid = threadIdx.x;
-    if (ROOT) {
+    if (ROOT && (((uintptr_t)bins_fm | (uintptr_t)ld_fm) & 15u) == 0) {
         static_assert(TPT == 16, "a thread's rows are one 16-byte load");
         if (tid * 16 < tn)
             *reinterpret_cast<uint4*>(s_bin + tid * 16) =
@@ -414,7 +415,9 @@ __device__ __forceinline__ void tile_bins(const uint8_t* __restrict__ bins_fm, i
 #pragma unroll 2
     for (int j = 0; j < TPT; ++j) {
         const int x = j * RB + tid;
-        if (x < tn) s_bin[x] = bins_rm[(size_t)crow[t0 + x] * (size_t)ld_rm + f];
+        if (x < tn)
+            s_bin[x] = ROOT ? bins_fm[(size_t)f * (size_t)ld_fm + (size_t)(t0 + x)]
+                            : bins_rm[(size_t)crow[t0 + x] * (size_t)ld_rm + f];
     }
 }
 
@@ -1423,11 +1426,14 @@ struct ChainRows {
     F32x4 g[CQ], h[CQ];
 };
 // And of its lists: entries CPT slot .. CPT slot + CPT - 1, the group's range.
+struct __attribute__((packed, aligned(2))) Pos8 {    // CPT positions, one load: the root table may lie at any position's address
+    uint32_t w[4];
+};
 struct ChainList {
-    uint4 idx;
+    Pos8 idx;
     uint32_t k0, k1;
 };
-static_assert(CPT * sizeof(uint16_t) == sizeof(uint4), "a thread's list entries are one load");
+static_assert(CPT * sizeof(uint16_t) == sizeof(Pos8), "a thread's list entries are one load");
 
 // Dense chains (no default bins), cgrow's row-order fp32 sums (grow.c:55-59);
 // the count cell is its chain of 1.0f adds, min(count, 2^24).  Block (feature
@@ -1546,14 +1552,14 @@ __global__ void __launch_bounds__(2 * CB) k_tile_chain(const float* __restrict__
         };
         auto load_list = [&](ChainList& c, int64_t t) {
             t = min(t, tiles - 1);
-            c.idx = *reinterpret_cast<const uint4*>(pf + t * WT + CPT * tid);   // entries past the rows: anything
+            c.idx = *reinterpret_cast<const Pos8*>(pf + t * WT + CPT * tid);   // entries past the rows: anything
             c.k0 = sf[(size_t)t * ST + b0];
             c.k1 = sf[(size_t)t * ST + b0 + w];
         };
         load_rows(rows[0], 0);
         load_rows(rows[1], 1);
         load_list(list[0], 0);
-        list[1].idx = make_uint4(0, 0, 0, 0);
+        list[1].idx = Pos8{{0, 0, 0, 0}};
         list[1].k0 = list[1].k1 = 0;
         // steps past the last tile repeat it, into cells that nothing reads
         const int64_t steps = (tiles + 1) / 2 * 2 + 2;
@@ -1565,7 +1571,7 @@ __global__ void __launch_bounds__(2 * CB) k_tile_chain(const float* __restrict__
                 const uint32_t at = CPT * tid;
                 ChainList& l = list[k ^ 1];
                 if (at + CPT > l.k0 && at < l.k1) {
-                    const uint32_t iw[4] = {l.idx.x, l.idx.y, l.idx.z, l.idx.w};
+                    const uint32_t iw[4] = {l.idx.w[0], l.idx.w[1], l.idx.w[2], l.idx.w[3]};
                     float2 v[CPT];
 #pragma unroll
                     for (int j = 0; j < CPT; ++j) v[j] = s_gh[k ^ 1][4 + ((iw[j / 2] >> (16 * (j & 1))) & (WT - 1))];
