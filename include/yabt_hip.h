@@ -265,7 +265,7 @@ int yabt_leaf_step(int x_kind, const void *X, int64_t ldx, int64_t n, int F, int
                    int64_t *out_count, float *out_value, float *out_linear, int32_t *out_status,
                    yabt_stream_t stream);
 
-/* Workspace bytes of yabt_leaf_moments for n rows. */
+/* Workspace bytes of yabt_leaf_moments for n rows, and enough for fewer. */
 size_t yabt_leaf_moments_workspace_bytes(int64_t n);
 
 /* Standardisation of the leaf-model inputs: out_mu[j] = mean, out_sd[j] =

@@ -93,6 +93,20 @@ def test_reference_root_order_sizes():
     assert rc < 0 and "bad pointer" in _lib.last_error()
 
 
+def test_leaf_moments_workspace_grows_with_the_rows():
+    """A buffer made for the largest row count is enough for the smaller ones,
+    and holds two doubles a model input (at most 8) of the row blocks: 1024 rows each,
+    more above 512 blocks, 16384 at most."""
+    lib = _lib.load()
+    sizes = sorted({max(1, b + d) for b in [1024 * k for k in range(1, 1100, 7)] + [524_288, 655_360, 2_000_000, 8_388_608]
+                    + [16_384 * k for k in range(500, 700, 3)] for d in (-1, 0, 1)})
+    got = [lib.yabt_leaf_moments_workspace_bytes(n) for n in sizes]
+    assert got == sorted(got)
+    for n, b in zip(sizes, got):
+        rows = min(max(-(-(-(-n // 512)) // 256) * 256, 1024), 16_384)
+        assert b >= 128 * -(-n // rows)
+
+
 def test_argument_errors_are_reported_without_a_device():
     lib = _lib.load()
     rc = lib.yabt_grow(None, 0, None, 0, None, None, None, None, ctypes.c_float(0.5), 0, None, None, None, 10, 0,

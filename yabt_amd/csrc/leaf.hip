@@ -1698,9 +1698,12 @@ int yabt_leaf_rank_features(const int64_t* feature, int n_nodes, int F, int k, i
     return launch_status("yabt_leaf_rank_features launch");
 }
 
+// The most blocks that any row count up to n takes, not n's own, which falls
+// where moment_rows grows: a buffer made for the largest n serves the smaller.
 size_t yabt_leaf_moments_workspace_bytes(int64_t n) {
     if (n < 0) return 0;
-    const int64_t mr = moment_rows(n), nb = n > 0 ? (n + mr - 1) / mr : 1;
+    const int64_t few = (n + MROWS_MIN - 1) / MROWS_MIN, many = std::max(MBLOCKS, (n + MROWS_MAX - 1) / MROWS_MAX);
+    const int64_t nb = std::max<int64_t>(1, std::min(few, many));
     const size_t f = (size_t)nb * 2 * LKMAX * sizeof(double), u = (size_t)MU8_BLOCKS * LKMAX * 2 * sizeof(uint64_t);
     return align_up(f > u ? f : u, 256);
 }
