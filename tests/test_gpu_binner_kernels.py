@@ -79,17 +79,13 @@ def test_fit_equals_numpy(n, missing):
     assert np.array_equal(b.medians_.view(np.uint32), np.nanmedian(X, axis=0).astype(np.float32).view(np.uint32))
 
 
-def test_medians_of_a_sample_that_is_not_random():
-    """The C entry takes any rows as the sample: the medians are of all rows."""
+def _medians(X, rows):
+    """yabt_bin_fit's medians of X from a caller's own sample."""
     import ctypes
     from yabt_amd import _lib
-    rng = np.random.default_rng(5)
-    n, F, m = 30_000, 300, 5000
-    X = rng.normal(size=(n, F)).astype(np.float32)
-    X = np.sort(X, axis=0)
-    X[:, 7] = np.nan
+    (n, F), m = X.shape, len(rows)
     dev = torch.device("cuda", 0)
-    Xd, rows = torch.from_numpy(X).to(dev), torch.arange(m, device=dev)     # the smallest values
+    Xd, rows = torch.from_numpy(X).to(dev), torch.from_numpy(rows).to(dev)
     lib = _lib.load()
     nb = int(lib.yabt_bin_fit_workspace_bytes(m, F))
     ws = torch.empty(nb, dtype=torch.uint8, device=dev)
@@ -98,7 +94,32 @@ def test_medians_of_a_sample_that_is_not_random():
     p = lambda t: ctypes.c_void_p(t.data_ptr())
     _lib.check(lib.yabt_bin_fit(p(Xd), F, n, F, p(rows), m, 256, p(ws), nb, p(edges), 255, p(ne), p(sc), p(med),
                                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "yabt_bin_fit")
+    return med.cpu().numpy()
+
+
+def test_medians_of_a_sample_that_is_not_random():
+    """The C entry takes any rows as the sample: the medians are of all rows."""
+    rng = np.random.default_rng(5)
+    n, F, m = 30_000, 300, 5000
+    X = rng.normal(size=(n, F)).astype(np.float32)
+    X = np.sort(X, axis=0)
+    X[:, 7] = np.nan
+    med = _medians(X, np.arange(m))                                        # the smallest values
     want = np.zeros(F, np.float32)
     keep = np.arange(F) != 7
     want[keep] = np.median(X[:, keep], axis=0)
-    assert np.array_equal(med.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(med.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("n,m", [(300_000, 2000), (300_001, 40), (50_000, 1), (40_000, 9000)])
+def test_medians_where_few_features_have_a_bracket(n, m):
+    """A sample so small that the rows around the median would not fit its
+    lists (no bracket), beside columns of ties (a bracket) and one whose sample is
+    all NaN (a bracket that misses), over two tiles of the select."""
+    rng = np.random.default_rng(n)
+    rows = rng.choice(n, m, replace=False)
+    X = np.stack([_column(rng, KINDS[f % len(KINDS)], n) for f in range(20)], axis=1)
+    X[rows, 17] = np.nan
+    X[rng.random(n) < 0.3, 4] = np.nan
+    med = _medians(X, rows)
+    assert np.array_equal(med.view(np.uint32), np.nanmedian(X, axis=0).astype(np.float32).view(np.uint32))

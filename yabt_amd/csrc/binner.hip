@@ -55,7 +55,7 @@ struct Bracket {
     uint32_t eq_lo, eq_hi; // rows with key lo, and key hi (> lo)
     uint32_t inside;       // rows between: list entries wanted (may exceed the list)
     uint32_t valid;        // non-NaN rows
-    uint32_t pad;
+    uint32_t missed;       // the two middle values are not among them: select over all rows
 };
 
 struct FitWs {
@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(TB) k_quantiles(const uint32_t* __restrict__ s
                                                   float* __restrict__ out_edges, int64_t ld_edges,
                                                   int32_t* __restrict__ out_nedges, float* __restrict__ out_scales,
                                                   float* __restrict__ out_medians, uint32_t* __restrict__ need_std,
-                                                  Bracket* __restrict__ br, uint32_t* __restrict__ missed) {
+                                                  Bracket* __restrict__ br, uint32_t* __restrict__ missed, int64_t n) {
     __shared__ float s_q[TB];
     __shared__ int s_wave[TB / WAVE];
     __shared__ int64_t s_lo, s_hi;
@@ -363,6 +363,26 @@ __global__ void __launch_bounds__(TB) k_quantiles(const uint32_t* __restrict__ s
         need_std[f] = s == 0.0;
         out_scales[f] = (float)s;
     }
+    Bracket bk = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+    if (!whole && c > 0) {
+        // the rows' median lies within 3 sqrt(c) sample ranks of the sample's
+        // (six standard deviations of a random sample's)
+        const int64_t mid = (c - 1) / 2, w = (int64_t)(3.0 * sqrt((double)c)) + 8;
+        const uint32_t lo = mid >= w ? sk[mid - w] : 0u, hi = mid + 1 + w < c ? sk[mid + 1 + w] : NAN_KEY - 1;
+        // the rows between the ends go into a list of m keys, n / m of them for
+        // each of the sample's, and two standard deviations more.  A list that
+        // would not hold them is not begun (the ends stay equal, at no value's
+        // key): keys that overflow it cost an atomic each on one counter (1M x
+        // 50, a sample of 2000: 1909 us with the list, 935 without; 990 by
+        // counting and selecting alone)
+        int in = 0;
+        for (int64_t i = max(mid - w, (int64_t)-1) + 1 + tid; i < min(mid + 1 + w, c); i += TB) in += sk[i] > lo && sk[i] < hi;
+        const double between = block_sum<TB, int>(in, s_wave);
+        if ((double)n * (between + 2.0 * sqrt(between)) <= (double)m * (double)m) {
+            bk.lo = lo;
+            bk.hi = hi;
+        }
+    }
     if (tid == 1) {
         if (whole) {
             // np.nanmedian of the rows, 0 where all are NaN (binning.py:32-33)
@@ -374,15 +394,7 @@ __global__ void __launch_bounds__(TB) k_quantiles(const uint32_t* __restrict__ s
             }
             out_medians[f] = med;
         } else {
-            // the rows' median lies within 3 sqrt(c) sample ranks of the
-            // sample's (six standard deviations of a random sample's)
-            Bracket b = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-            if (c > 0) {
-                const int64_t mid = (c - 1) / 2, w = (int64_t)(3.0 * sqrt((double)c)) + 8;
-                b.lo = mid >= w ? sk[mid - w] : 0u;
-                b.hi = mid + 1 + w < c ? sk[mid + 1 + w] : NAN_KEY - 1;
-            }
-            br[f] = b;
+            br[f] = bk;
         }
     }
     if (f == 0 && tid == 2) *missed = 0;
@@ -506,9 +518,12 @@ __global__ void __launch_bounds__(ST) k_std_scale(const uint32_t* __restrict__ o
 
 // One pass over X, every thread one feature (neighbouring threads neighbouring
 // features): rows below, at and between the bracket's ends; the keys between
-// go into the feature's list (cap places).  About 6 sqrt(c) / c of the rows lie
-// between (1.3% at a sample of 200 000), whatever ties there are: a value that
-// holds more of them than that is an end of the bracket.  2M x 50: 215 us (1.9
+// go into the feature's list (cap places).  At most about 6 sqrt(c) / c of the
+// rows lie between (1.35% at a sample of 200 000, fewer where values are tied:
+// one that holds more of them than that is an end of the bracket); a list of a
+// sample's size holds them up to 14.3M rows without ties, and k_quantiles
+// gives no bracket to a feature whose rows it would not hold: these rows are
+// only counted.  2M x 50: 215 us (1.9
 // TB/s of X) and 23 us for the lists' selects; counting the numbers and
 // four digit passes over X took 1580 us and 170 us of steps between them.
 constexpr int MT = 256;                        // threads
@@ -576,7 +591,7 @@ __global__ void __launch_bounds__(MT) k_median_pass(const float* __restrict__ X,
 
 // One block per feature: the two middle order statistics from the counts and
 // the list (a radix select of the list's keys), or *missed.
-__global__ void __launch_bounds__(1024) k_median_finish(const Bracket* __restrict__ br, const uint32_t* __restrict__ lists,
+__global__ void __launch_bounds__(1024) k_median_finish(Bracket* __restrict__ br, const uint32_t* __restrict__ lists,
                                                         int64_t cap, uint32_t* __restrict__ cnt,
                                                         uint32_t* __restrict__ missed, float* __restrict__ out_medians) {
     __shared__ uint32_t s_h[2][NB];
@@ -600,7 +615,10 @@ __global__ void __launch_bounds__(1024) k_median_finish(const Bracket* __restric
         else miss = true;
     }
     if (miss) {
-        if (tid == 0) *missed = 1;
+        if (tid == 0) {
+            br[f].missed = 1;
+            *missed = 1;
+        }
         return;
     }
     if (search) {
@@ -667,9 +685,10 @@ __global__ void __launch_bounds__(1024) k_median_finish(const Bracket* __restric
 }
 
 // ---------------------------------------------------------------------------
-// medians over all rows: radix select of the two middle order statistics, run
-// where a bracket missed (a sample that is no random one); every kernel here
-// ends at once otherwise
+// medians over all rows: radix select of the two middle order statistics, for
+// the features whose bracket missed (a sample that is no random one) or that got
+// none (k_quantiles: more rows than their list holds); every kernel here ends
+// at once where there is no such feature
 // ---------------------------------------------------------------------------
 
 // state[f][t] = {prefix, rank}: the ranks of the two middle order statistics.
@@ -688,17 +707,19 @@ __global__ void k_select_init(const uint32_t* __restrict__ missed, const uint32_
 }
 
 // Histogram of digit `shift` among keys whose higher bits equal each target's prefix.
-__global__ void __launch_bounds__(TB) k_select_hist(const uint32_t* __restrict__ missed, const float* __restrict__ X,
-                                                    int64_t ldx, int64_t n, int F, int shift,
+__global__ void __launch_bounds__(TB) k_select_hist(const uint32_t* __restrict__ missed, const Bracket* __restrict__ br,
+                                                    const float* __restrict__ X, int64_t ldx, int64_t n, int F, int shift,
                                                     const uint32_t* __restrict__ state, uint32_t* __restrict__ hist) {
     __shared__ uint32_t s_h[HT][2][NB];
     if (!*missed) return;
     const int f0 = blockIdx.y * HT;
-    for (int i = threadIdx.x; i < HT * 2 * NB; i += TB) (&s_h[0][0][0])[i] = 0;
-    __syncthreads();
     const int j = threadIdx.x % HT;
     const int f = f0 + j;
-    if (f < F) {
+    const bool mine = f < F && br[f].missed;
+    if (!__syncthreads_or(mine)) return;
+    for (int i = threadIdx.x; i < HT * 2 * NB; i += TB) (&s_h[0][0][0])[i] = 0;
+    __syncthreads();
+    if (mine) {
         const uint32_t p1 = state[(size_t)f * 4 + 0], p2 = state[(size_t)f * 4 + 2];
         for (int64_t r = (int64_t)blockIdx.x * (TB / HT) + threadIdx.x / HT; r < n; r += (int64_t)gridDim.x * (TB / HT)) {
             const float v = X[(size_t)r * ldx + f];
@@ -739,10 +760,11 @@ __global__ void k_select_step(const uint32_t* __restrict__ missed, int F, uint32
 
 // median = x_k (odd count) or float32 (x_k1 + x_k2) / 2 (even), 0 if no value
 // (np.nanmedian then np.where(isnan, 0, .), binning.py:32-33).
-__global__ void k_select_finish(const uint32_t* __restrict__ missed, const uint32_t* __restrict__ cnt, int F,
-                                const uint32_t* __restrict__ state, float* __restrict__ out_medians) {
+__global__ void k_select_finish(const uint32_t* __restrict__ missed, const Bracket* __restrict__ br,
+                                const uint32_t* __restrict__ cnt, int F, const uint32_t* __restrict__ state,
+                                float* __restrict__ out_medians) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= F || !*missed) return;
+    if (f >= F || !*missed || !br[f].missed) return;
     const uint32_t c = cnt[f];
     float med = 0.0f;
     if (c > 0) {
@@ -952,7 +974,7 @@ int yabt_bin_fit(const float* X, int64_t ldx, int64_t n, int F, const int64_t* s
     }
     const int whole = !sample_rows;            // the sample is all rows
     k_quantiles<<<F, TB, 0, stream>>>(w.ka, m, max_bins, whole, out_edges, ld_edges, out_nedges, out_scales, out_medians,
-                                      w.need_std, w.br, w.missed);
+                                      w.need_std, w.br, w.missed, n);
     k_std_scale<<<F, ST, 0, stream>>>(w.orig, reinterpret_cast<float*>(w.kb), m, w.need_std, out_scales);
     if (whole) return launch_status("yabt_bin_fit launch");
     // medians over all n rows
@@ -963,10 +985,10 @@ int yabt_bin_fit(const float* X, int64_t ldx, int64_t n, int F, const int64_t* s
     const dim3 grid((unsigned)launch_grid(max(n, (int64_t)1), TB / HT * 8, 1024), (unsigned)((F + HT - 1) / HT));
     k_select_init<<<(F + 63) / 64, 64, 0, stream>>>(w.missed, w.cnt, F, w.sel_state, w.sel_hist);
     for (int shift = 24; shift >= 0; shift -= 8) {
-        k_select_hist<<<grid, TB, 0, stream>>>(w.missed, X, ldx, n, F, shift, w.sel_state, w.sel_hist);
+        k_select_hist<<<grid, TB, 0, stream>>>(w.missed, w.br, X, ldx, n, F, shift, w.sel_state, w.sel_hist);
         k_select_step<<<(F + 63) / 64, 64, 0, stream>>>(w.missed, F, w.sel_state, w.sel_hist);
     }
-    k_select_finish<<<(F + 63) / 64, 64, 0, stream>>>(w.missed, w.cnt, F, w.sel_state, out_medians);
+    k_select_finish<<<(F + 63) / 64, 64, 0, stream>>>(w.missed, w.br, w.cnt, F, w.sel_state, out_medians);
     return launch_status("yabt_bin_fit launch");
 }
 
