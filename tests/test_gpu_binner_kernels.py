@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,F,longest", [
     (1, 1, 255), (15, 60, 1), (255, 61, 255), (256, 4, 128), (257, 60, 127), (1000, 121, 255), (300, 500, 30),
     (70001, 2, 254), (600, 17, 0),
+    (2_100_003, 1, 200), (530_001, 4, 255), (9001, 13, 100), (270_001, 29, 64),   # tiles of 4096 rows down to 16
 ])
 def test_transform_equals_searchsorted(n, F, longest):
     rng = np.random.default_rng(n + F)

@@ -779,31 +779,44 @@ __global__ void k_select_finish(const uint32_t* __restrict__ missed, const Brack
 // transform
 // ---------------------------------------------------------------------------
 
-// A block keeps its feature group's edges in LDS and takes tiles of TR rows:
+// A block keeps its feature group's edges in LDS and takes tiles of tr rows:
 //   * a tile's values are read in memory order (lanes over neighbouring
 //     features), imputed and stored the same way, and each looked up by its lane
 //     in its own feature's edges.  The edges lie as a complete search tree
 //     in level order (node k's children 2k and 2k + 1; +inf where a feature
-//     has fewer edges), so a lookup is one read, compare and add a level, as
-//     many levels as the group's longest edge list needs; tables of different
-//     features start a bank apart;
+//     has fewer edges), so a lookup is one read, compare and add a level; it
+//     starts at the root of the leftmost subtree that holds the group's longest
+//     edge list, so its levels are as many as that list needs.  Tables of
+//     different features start a bank apart;
 //   * the bins wait in LDS as [feature][row] bytes and leave as 16 rows of a
 //     feature (feature-major) and as 4 x 4 blocks turned into 4 features of a
 //     row (row-major), both in whole lines.
-// Bound by HBM (X in, two byte layouts and the imputed matrix out: 1.03 GB at
-// 2M x 50) and the lookups' LDS reads: 2684 -> 365 us there (2.8 TB/s).  A row
-// per thread, as before, read X at the row stride and searched sorted edges
-// at addresses that share four of the 64 banks.
+// 2684 -> 365 us at 2M x 50 (X in, two byte layouts and the imputed matrix out:
+// 1.03 GB, 2.8 TB/s, under half of a copy's rate): a tile's loads, its lookups'
+// LDS reads and its stores follow one another, over the 16 waves a CU that the
+// tables leave.  A row per thread, as before, read X at the row stride and
+// searched sorted edges at addresses that share four of the 64 banks.
 constexpr int TT = 512;                        // threads of a transform block
-constexpr int TR = 256;                        // rows per tile
+constexpr int TL = 8;                          // levels of a table: MAXE edges
 constexpr int TSTRIDE = NB + 1;                // words between two features' tables
-constexpr int TBYTES = TR + 4;                 // bytes between two features' bins
 constexpr int TFEAT = 60;                      // features per block: two blocks' LDS on a CU
+// Values of a tile, at most: with few features a tile of more rows, so that
+// every thread has several values in flight between two barriers.
+constexpr int TVALUES = 16384;
+
+// log2 of a tile's rows: TVALUES / fg of them, halved (down to 16, and to a
+// value a thread) while the tiles are not two blocks a CU.
+inline int transform_rows_log2(int64_t n, int F, int fg, int groups) {
+    int l = 4;
+    while ((fg << (l + 1)) <= TVALUES) ++l;
+    while (l > 4 && (std::min(F, fg) << l) > TT && ((n + (1ll << l) - 1) >> l) * groups < 512) --l;
+    return l;
+}
 
 struct TransformArgs {
     const float* X;
     int64_t ldx, n;
-    int F, fg;                                 // fg: features per group (a multiple of 4)
+    int F, fg, trl;                            // fg: features per group (a multiple of 4); trl: log2 of a tile's rows
     const float* edges;
     int64_t ld_edges;
     const int32_t* nedges;
@@ -819,35 +832,36 @@ struct TransformArgs {
 
 __global__ void __launch_bounds__(TT) k_transform(TransformArgs A) {
     extern __shared__ char smem[];
-    __shared__ int s_levels;
+    __shared__ int s_any;                                              // the group's edge counts, or-ed
+    const int tr = 1 << A.trl, bstride = tr + 4;                       // bytes between two features' bins
     float* s_e = reinterpret_cast<float*>(smem);                       // [fg][TSTRIDE]
     float* s_med = s_e + A.fg * TSTRIDE;                               // [fg]
-    uint8_t* s_b = reinterpret_cast<uint8_t*>(s_med + A.fg);           // [fg][TBYTES]
+    uint8_t* s_b = reinterpret_cast<uint8_t*>(s_med + A.fg);           // [fg][bstride]
     const int f0 = blockIdx.y * A.fg, nf = min(A.fg, A.F - f0);
     const int tid = threadIdx.x;
-    if (tid == 0) s_levels = 0;
+    if (tid == 0) s_any = 0;
     __syncthreads();
-    for (int j = tid; j < nf; j += TT) {
-        const int ne = min(max(A.nedges[f0 + j], 0), MAXE);
-        atomicMax(&s_levels, ne ? 32 - __clz(ne) : 0);
-        s_med[j] = A.medians[f0 + j];
+    if (tid < nf) {
+        atomicOr(&s_any, min(max(A.nedges[f0 + tid], 0), MAXE));
+        s_med[tid] = A.medians[f0 + tid];
     }
-    __syncthreads();
-    const int levels = s_levels, nodes = 1 << levels;
-    for (int i = tid; i < nf * nodes; i += TT) {
-        const int j = i >> levels, k = i & (nodes - 1);
+    // edges and edge counts are read together: an edge past its list is not used
+#pragma unroll 4
+    for (int i = tid; i < nf << TL; i += TT) {
+        const int j = i >> TL, k = i & (NB - 1);
         if (k == 0) continue;
         const int lv = 31 - __clz(k);                                  // node k: number k - 2^lv of level lv
-        const int at = ((2 * (k - (1 << lv)) + 1) << (levels - 1 - lv)) - 1;
-        const int ne = min(max(A.nedges[f0 + j], 0), MAXE);
-        s_e[j * TSTRIDE + k] = at < ne ? A.edges[(size_t)(f0 + j) * A.ld_edges + at] : INFINITY;
+        const int at = ((2 * (k - (1 << lv)) + 1) << (TL - 1 - lv)) - 1;
+        const float e = A.edges[(size_t)(f0 + j) * A.ld_edges + min((int64_t)at, A.ld_edges - 1)];
+        s_e[j * TSTRIDE + k] = at < min(max(A.nedges[f0 + j], 0), MAXE) ? e : INFINITY;
     }
+    __syncthreads();
+    const int levels = __builtin_amdgcn_readfirstlane(s_any ? 32 - __clz(s_any) : 0), root = NB >> levels;
     // the bins of the row-major layout's columns up to the next multiple of 16 are zero
     const int last = blockIdx.y + 1 == gridDim.y;
     const int nq = last && A.rm_vec ? (((A.F + 15) & ~15) - f0) / 4 : (nf + 3) / 4;
-    for (int64_t r0 = (int64_t)blockIdx.x * TR; r0 < A.n; r0 += (int64_t)gridDim.x * TR) {
-        const int rows = (int)min((int64_t)TR, A.n - r0);
-        __syncthreads();                       // the tables; the last tile's bins are out
+    for (int64_t r0 = (int64_t)blockIdx.x << A.trl; r0 < A.n; r0 += (int64_t)gridDim.x << A.trl) {
+        const int rows = (int)min((int64_t)tr, A.n - r0);
         const int total = rows * nf, dj = TT % nf, dr = TT / nf;
         constexpr int U = 4;
         int j = tid % nf, r = tid / nf;
@@ -873,7 +887,7 @@ __global__ void __launch_bounds__(TT) k_transform(TransformArgs A) {
             for (int u = 0; u < U; ++u) {
                 if (isnan(x[u])) x[u] = s_med[jj[u]];
                 if (A.imp && i0 + u * TT < total) A.imp[(size_t)(r0 + rr[u]) * A.ld_imp + f0 + jj[u]] = x[u];
-                k[u] = 1;
+                k[u] = root;
                 e[u] = s_e + jj[u] * TSTRIDE;
             }
             for (int lv = 0; lv < levels; ++lv) {
@@ -882,29 +896,35 @@ __global__ void __launch_bounds__(TT) k_transform(TransformArgs A) {
             }
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                if (i0 + u * TT < total) s_b[jj[u] * TBYTES + rr[u]] = (uint8_t)(k[u] - nodes);
+                if (i0 + u * TT < total) s_b[jj[u] * bstride + rr[u]] = (uint8_t)(k[u] - NB);
         }
         __syncthreads();
         if (A.fm) {
-            for (int i = tid; i < nf * (TR / 16); i += TT) {
-                const int jf = i / (TR / 16), r16 = (i % (TR / 16)) * 16;
+            for (int i = tid; i < nf << (A.trl - 4); i += TT) {
+                const int jf = i >> (A.trl - 4), r16 = (i & ((tr >> 4) - 1)) * 16;
                 if (r16 >= rows) continue;
-                const uint32_t* src = reinterpret_cast<const uint32_t*>(s_b + jf * TBYTES + r16);
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(s_b + jf * bstride + r16);
                 uint8_t* dst = A.fm + (size_t)(f0 + jf) * A.ld_fm + r0 + r16;
                 if (A.fm_vec && r16 + 16 <= rows) {
                     *reinterpret_cast<uint4*>(dst) = make_uint4(src[0], src[1], src[2], src[3]);
                 } else {
-                    for (int q = 0; q < 16 && r16 + q < rows; ++q) dst[q] = s_b[jf * TBYTES + r16 + q];
+                    for (int q = 0; q < 16 && r16 + q < rows; ++q) dst[q] = s_b[jf * bstride + r16 + q];
                 }
             }
         }
-        if (A.rm && A.rm_vec) {
-            for (int i = tid; i < nq * (TR / 4); i += TT) {
+        if (A.rm && A.rm_vec && nf <= 4 && nq == 4) {      // a row is 16 bytes: one store
+            for (int i = tid; i < rows; i += TT) {
+                uint32_t w = 0;
+                for (int t = 0; t < nf; ++t) w |= (uint32_t)s_b[t * bstride + i] << (8 * t);
+                *reinterpret_cast<uint4*>(A.rm + (size_t)(r0 + i) * A.ld_rm + f0) = make_uint4(w, 0u, 0u, 0u);
+            }
+        } else if (A.rm && A.rm_vec) {
+            for (int i = tid; i < nq * (tr / 4); i += TT) {
                 const int q = i % nq, r4 = (i / nq) * 4;
                 uint32_t c[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
-                    c[t] = 4 * q + t < nf ? *reinterpret_cast<const uint32_t*>(s_b + (4 * q + t) * TBYTES + r4) : 0u;
+                    c[t] = 4 * q + t < nf ? *reinterpret_cast<const uint32_t*>(s_b + (4 * q + t) * bstride + r4) : 0u;
                 // byte t of row t4's word: byte t4 of feature t's word
                 const uint32_t a0 = __builtin_amdgcn_perm(c[1], c[0], 0x05010400u), a1 = __builtin_amdgcn_perm(c[1], c[0], 0x07030602u);
                 const uint32_t b0 = __builtin_amdgcn_perm(c[3], c[2], 0x05010400u), b1 = __builtin_amdgcn_perm(c[3], c[2], 0x07030602u);
@@ -918,7 +938,7 @@ __global__ void __launch_bounds__(TT) k_transform(TransformArgs A) {
         } else if (A.rm) {
             int jb = tid % nf, rb = tid / nf;
             for (int i = tid; i < total; i += TT) {
-                A.rm[(size_t)(r0 + rb) * A.ld_rm + f0 + jb] = s_b[jb * TBYTES + rb];
+                A.rm[(size_t)(r0 + rb) * A.ld_rm + f0 + jb] = s_b[jb * bstride + rb];
                 jb += dj;
                 rb += dr;
                 if (jb >= nf) {
@@ -927,6 +947,7 @@ __global__ void __launch_bounds__(TT) k_transform(TransformArgs A) {
                 }
             }
         }
+        __syncthreads();                       // the tile's bins are out
     }
 }
 
@@ -1001,15 +1022,16 @@ int yabt_bin_transform(const float* X, int64_t ldx, int64_t n, int F, const floa
     if (!X || !edges || !nedges || !medians || !(out_fm || out_rm || out_imputed))
         return fail(-2, "yabt_bin_transform: null pointer argument");
     if (n == 0) return 0;
-    const int groups = (F + TFEAT - 1) / TFEAT;
-    const int fg = ((F + groups - 1) / groups + 3) / 4 * 4;
+    const int even = (F + TFEAT - 1) / TFEAT, fg = ((F + even - 1) / even + 3) / 4 * 4, groups = (F + fg - 1) / fg;
+    const int trl = transform_rows_log2(n, F, fg, groups);
     // 16-byte row stores when every 16-feature tile of every row is 16-byte aligned
-    const TransformArgs A{X, ldx, n, F, fg, edges, ld_edges, nedges, medians, out_fm, ld_fm, out_rm, ld_rm, out_imputed,
+    const TransformArgs A{X, ldx, n, F, fg, trl, edges, ld_edges, nedges, medians, out_fm, ld_fm, out_rm, ld_rm, out_imputed,
                           ld_imputed, out_fm && ld_fm % 16 == 0 && aligned16(out_fm),
                           out_rm && ld_rm % 16 == 0 && aligned16(out_rm)};
-    const size_t lds = (size_t)fg * (TSTRIDE * 4 + 4 + TBYTES);
-    // two blocks a CU stay for all tiles: each loads its edges once
-    const dim3 grid((unsigned)launch_grid(n, TR, std::max(1, 512 / ((F + fg - 1) / fg))), (unsigned)((F + fg - 1) / fg));
+    const size_t lds = (size_t)fg * (TSTRIDE * 4 + 4 + (1 << trl) + 4);
+    // as many blocks as are resident stay for all tiles: each loads its edges once
+    const int resident = 256 * (int)std::min<size_t>(2048 / TT, 160 * 1024 / (lds + 64));
+    const dim3 grid((unsigned)launch_grid(n, 1 << trl, std::max(1, resident / groups)), (unsigned)groups);
     k_transform<<<grid, TT, lds, stream>>>(A);
     return launch_status("yabt_bin_transform launch");
 }
