@@ -332,8 +332,9 @@ size_t yabt_grow_levelwise_workspace_bytes(int64_t n, int F, int max_leaves, int
  * leaf table (yabt/_cgrow/grow.c:321-408) over the computed gains.  Same
  * arguments and outputs as yabt_grow (no default_bin) -- bit-identical node
  * arrays -- plus out_leaf_of_row (n int64, may be NULL): each row's leaf.
- * Returns -3 if the budget could bind.  One device round trip per depth;
- * the call synchronises `stream`. */
+ * Returns -3 if the budget could bind.  The host enqueues the depths, at most
+ * two past the last one whose splits it has seen, and the call synchronises
+ * `stream`. */
 int yabt_grow_levelwise(const uint8_t *bins_fm, int64_t ld_fm, const uint8_t *bins_rm, int64_t ld_rm,
                         const float *grad, const float *hess, const uint8_t *fmask, const float *imat,
                         float ib, int use_imat, const int32_t *nbins, const uint32_t *bin_counts,

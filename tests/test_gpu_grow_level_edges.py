@@ -39,6 +39,37 @@ def test_depth_batched_equals_sequential(n, F, nb, depth, msl, const_h, outlier)
     assert torch.equal(a.leaf_of_row, b.leaf_of_row)
 
 
+@pytest.mark.parametrize("n,F,depth,gamma,most", [
+    (1000, 5, 15, 1e9, 0),          # the root does not split: 32768 places for one node
+    (20_000, 20, 15, 20.0, 0),      # a few splits, the deepest far above the cap
+    (3000, 3, 1, 0.0, 0),           # the cap itself ends it
+    (50_000, 6, 10, 5.0, 0),
+    (300_000, 4, 15, 0.0, 4097),    # more splits of one depth than the LDS counters, the pick's and the scan's blocks
+])
+def test_work_follows_the_splits_that_exist(n, F, depth, gamma, most):
+    """Growth that ends far above its cap, and depths with so many splits that
+    the launches go over them in strides: split-by-split growth's tree."""
+    dev = torch.device("cuda", 0)
+    rng = np.random.default_rng(n + depth)
+    bins = torch.from_numpy(rng.integers(0, 256, size=(n, F)).astype(np.uint8)).to(dev)
+    signal = bins.float().sum(1) / 64 if most else (bins[:, 0] > 99).float()     # the first: even splits
+    g = signal + torch.from_numpy(rng.normal(size=n).astype(np.float32)).to(dev)
+    h = torch.ones(n, device=dev)
+    lay = G.make_layouts(bins, dev)
+    kw = dict(max_leaves=2 ** depth, max_depth=depth, msl=1, mcw=0.0, gamma=gamma, lam=0.0 if most else 1.0)
+    a = G.grow_device(lay, g, h, np.full(F, 256, np.int32), growth="levelwise", **kw)
+    kw["max_leaves"] = min(kw["max_leaves"], 32767)      # which no tree here reaches
+    b = G.grow_device(lay, g, h, np.full(F, 256, np.int32), growth="sequential", **kw)
+    assert a.n_nodes == b.n_nodes < 2 * 32767 - 1
+    for k in ("feature", "thr_bin", "left", "right", "depth"):
+        assert torch.equal(getattr(a, k), getattr(b, k)), k
+    assert torch.equal(a.value.view(torch.int32), b.value.view(torch.int32))
+    assert torch.equal(a.leaf_of_row, b.leaf_of_row)
+    if most:
+        splits = torch.bincount(a.depth[a.feature >= 0], minlength=depth)
+        assert int(splits[:depth - 1].max()) >= most
+
+
 def test_depth_batched_reports_non_finite():
     dev = torch.device("cuda", 0)
     lay = G.make_layouts(torch.zeros((100, 2), dtype=torch.uint8, device=dev), dev)
