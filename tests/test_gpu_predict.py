@@ -104,6 +104,18 @@ def numpy_predict(A, X, K, clamp, start):
     (66000, 9, 6, [700, 3], 8, True, {}),                              # trees larger than the LDS
     (4097, 500, 30, [31], 8, True, {2: "child"}),                      # rows too wide for the LDS
     (4097, 200, 1, [31], 8, False, {}),                                # too few trees to stage wide rows
+    (4097, 200, 2, [31], 8, False, {}),
+    (20_001, 12, 1, [31], 8, True, {}),                                # a row per thread: one tree,
+    (140_001, 90, 1, [31], 0, True, {0: "swapped"}),
+    (140_001, 16, 3, [31, 2], 0, True, {1: "cycle"}),                  # three on narrow rows,
+    (131_073, 300, 5, [31, 1], 0, True, {3: "child", 2: "feature"}),   # a few on wide ones
+    (2049, 20, 0, [1], 0, True, {}),                                   # no tree
+    (2049, 20, 75, [31, 1, 63], 0, True, {4: "child", 33: "cycle", 64: "swapped"}),   # constant leaves: tiles of 64,
+    (32_767, 40, 33, [9, 200], 0, True, {8: "feature"}),               # trees that would not leave places for the groups,
+    (4097, 500, 40, [31, 1], 0, True, {5: "cycle"}),                   # rows too wide for the LDS
+    (20_003, 60, 20, [300, 2], 0, True, {}),
+    (4099, 30, 20, [300, 5], 8, True, {2: "swapped"}),
+    (270_001, 110, 18, [63], 8, True, {}),                             # two rounds of blocks, 64 rows a tile
 ])
 def test_predict_equals_numpy(n, F, T, leaves, K, clamp, odd):
     import torch

@@ -111,16 +111,24 @@ __device__ __forceinline__ int64_t tree_nodes(const Forest& A, int t, int64_t* o
 
 // One row's walk through a tree in global memory, as capply does
 // (yabt/_cgrow/grow.c:223-239): it stops at a leaf, at an out-of-range
-// feature or child, or after as many steps as the tree has nodes.
-template <typename XF>
+// feature or child, or after as many steps as the tree has nodes.  BOTH: the
+// two children are loaded with the threshold, so that a step waits once; else
+// only the one taken, for narrow rows enough to hide the waits (1M x 10, 1000
+// leaves: 67 and 62 us; x 28 112 and 139).
+template <bool BOTH = true, typename XF>
 __device__ int64_t walk_global(const Forest& A, int64_t off, int64_t nt, const XF& x) {
     int64_t node = 0;
     for (int64_t s = 0; s < nt; ++s) {
         const int64_t f = A.feature[off + node];
         if (f < 0 || f >= A.F) break;
         const float thr = A.threshold[off + node];
-        const int64_t l = A.left[off + node], r = A.right[off + node];   // both: the walk waits once a step
-        const int64_t nxt = (x((int)f) <= thr) ? l : r;
+        int64_t nxt;
+        if (BOTH) {
+            const int64_t l = A.left[off + node], r = A.right[off + node];
+            nxt = (x((int)f) <= thr) ? l : r;
+        } else {
+            nxt = (x((int)f) <= thr) ? A.left[off + node] : A.right[off + node];
+        }
         if (nxt < 0 || nxt >= nt) break;
         node = nxt;
     }
@@ -182,6 +190,24 @@ __global__ void __launch_bounds__(BB) k_predict_rows(Forest A, const float* __re
     if (threadIdx.x == 0) out[i] = acc;
 }
 
+// Rows enough but little work in each (predict_flat): a row per thread, the trees
+// in order.
+template <bool BOTH>
+__global__ void __launch_bounds__(BB) k_predict_flat(Forest A, const float* __restrict__ X, int64_t ldx, int64_t n, float base,
+                                                     int accumulate, float* __restrict__ out) {
+    for (int64_t i = (int64_t)blockIdx.x * BB + threadIdx.x; i < n; i += (int64_t)gridDim.x * BB) {
+        const float* row = X + (size_t)i * (size_t)ldx;
+        const auto x = [row](int f) { return row[f]; };
+        float acc = accumulate ? out[i] : base;
+        for (int t = 0; t < A.T; ++t) {
+            int64_t off;
+            const int64_t nt = tree_nodes(A, t, &off);
+            if (nt > 0) acc += node_output(A, t, walk_global<BOTH>(A, off, nt, x), x);
+        }
+        out[i] = acc;
+    }
+}
+
 // Many rows: a block takes up to PRED_TILES tiles of R rows and the forest in
 // batches of trees that fit its LDS; every tile walks a batch before the next
 // one is loaded.
@@ -200,8 +226,8 @@ __global__ void __launch_bounds__(BB) k_predict_rows(Forest A, const float* __re
 // on with its next tree instead of waiting for the deepest of the wave), two
 // such lists side by side; then the leaves' models are evaluated tree by tree,
 // and the outputs are added in tree order.  Trees whose nodes do not have that
-// form (children not neighbours or not after their parent, more nodes than
-// the LDS holds) are walked in global memory.
+// form (children not neighbours or not after their parent, more than tcap nodes)
+// are walked in global memory.
 //
 // 500 000 rows x 50 features, 200 trees of 63 leaves with 8 inputs: 1.41 ms
 // (0.63 ms without linear leaves), 18.9 ms by a walk per row and tree in
@@ -227,7 +253,7 @@ __device__ __forceinline__ float clamp_quiet(float x, float lo, float hi) {
 
 template <int R, int G, bool XLDS, bool LIN>
 __global__ void __launch_bounds__(R * G) k_predict_tile(Forest A, const float* __restrict__ X, int64_t ldx, int64_t n,
-                                                        int tiles, int tb, int ncap, int lcap, float base,
+                                                        int tiles, int tb, int ncap, int tcap, int lcap, float base,
                                                         int accumulate, float* __restrict__ out) {
     constexpr int NT = R * G;
     static_assert(!XLDS || NT >= 4 * R, "rows of a tile are staged by four threads each");
@@ -270,7 +296,7 @@ __global__ void __launch_bounds__(R * G) k_predict_tile(Forest A, const float* _
             const int t = t0 + tid;
             int64_t off = 0, nt = 0;
             if (tid < tb && t < A.T) nt = tree_nodes(A, t, &off);
-            const int fit = nt > 0 && nt <= ncap && A.F < 32767;
+            const int fit = nt > 0 && nt <= tcap && A.F < 32767;
             const int mine = fit ? (int)nt : 0;
             int sum = mine;
 #pragma unroll
@@ -472,10 +498,27 @@ size_t predict_lds(int R, bool xlds, bool lin, int F, int tiles, int tb, int nca
 
 constexpr size_t PRED_LDS = 156 * 1024;        // dynamic LDS of a tile block (one a CU)
 
+// Rows up to which a block per row is faster than tiles of rows: with 200
+// trees of 63 linear leaves, 50 features, 2048 rows take 94 us by blocks (46 us
+// per 1000 more) and 129 us by tiles (flat up to ~8000 rows, a tile a CU).
+constexpr int64_t PRED_ROW_BLOCKS = 2048;
+// Rows from which tiles of 256 (each stages the forest once per 256 rows or
+// more) beat tiles of 64 (four times as many blocks): 20 000 rows 187 us by
+// 64, 65 536 rows 234 us by 256.
+constexpr int64_t PRED_WIDE_ROWS = 32768;
+
+// Tiles of a block: one block a CU, in as many rounds of them as PRED_TILES asks,
+// all of the same size (300 000 rows x 100, 200 trees of 63 leaves: 1403 us in 293
+// blocks of 16 tiles, 961 in 469 of 10).
+inline int predict_tiles_per_block(int64_t n, int R) {
+    const int64_t slots = 256 * (int64_t)R, rounds = (n + slots * PRED_TILES - 1) / (slots * PRED_TILES);
+    return (int)((n + slots * rounds - 1) / (slots * rounds));
+}
+
 template <int R, int G, bool XLDS, bool LIN>
 int launch_predict(const Forest& A, const float* X, int64_t ldx, int64_t n, float base, int accumulate, float* out,
                    hipStream_t stream) {
-    const int tiles = (int)std::min<int64_t>(PRED_TILES, std::max<int64_t>(1, (n + 256 * R - 1) / (256 * R)));
+    const int tiles = predict_tiles_per_block(n, R);
     const int tb = std::min(LIN ? 16 : PRED_TB, std::max(A.T, 1));
     // half the nodes of a tree are leaves: two node places per leaf place
     const size_t fixed = predict_lds(R, XLDS, LIN, A.F, tiles, tb, 0, 0);
@@ -483,10 +526,20 @@ int launch_predict(const Forest& A, const float* X, int64_t ldx, int64_t n, floa
     lcap = std::min<int64_t>(std::min<int64_t>(lcap, 4096), std::max<int64_t>(A.n_total, 16));
     lcap = std::min<int64_t>(lcap, (int64_t)tb * R) & ~(int64_t)3;
     const int ncap = (int)(2 * lcap);
+    // Trees of which a batch holds too few for the groups leave threads idle, and the
+    // tile's inputs are read again for every batch: they are walked in global
+    // memory instead.  Constant leaves: 20 trees of 1000, 20 000 rows x 50 219 us
+    // one tree a batch, 59 walked; 300 000 x 300 14.4 ms, 0.94.  Linear leaves: 78
+    // trees of 255, 20 000 x 50 300 and 237 us; of 200, 16 trees, 200 000 x 100 280
+    // in LDS, four a batch, 340 walked.  Staged tiles of 256 rows fill their four
+    // groups or read few batches: 40 linear trees of 500, 300 000 x 10, 893 us in
+    // LDS, 1236 walked
+    const int least = G == 16 ? (!LIN ? 16 : n < PRED_WIDE_ROWS ? 8 : 4) : XLDS ? 1 : 4;
+    const int tcap = ncap / std::max(1, std::min(least, A.T));
     const size_t lds = predict_lds(R, XLDS, LIN, A.F, tiles, tb, ncap, (int)lcap);
     const int64_t per = (int64_t)tiles * R;
     k_predict_tile<R, G, XLDS, LIN><<<(unsigned)((n + per - 1) / per), R * G, lds, stream>>>(
-        A, X, ldx, n, tiles, tb, ncap, (int)lcap, base, accumulate, out);
+        A, X, ldx, n, tiles, tb, ncap, tcap, (int)lcap, base, accumulate, out);
     return launch_status("yabt_predict launch");
 }
 
@@ -497,26 +550,53 @@ int launch_predict(const Forest& A, const float* X, int64_t ldx, int64_t n, floa
                    : launch_predict<R, G, XLDS, false>(A, X, ldx, n, base, accumulate, out, stream);
 }
 
-// Rows up to which a block per row is faster than tiles of rows: with 200
-// trees of 63 linear leaves, 50 features, 2048 rows take 94 us by blocks (46 us
-// per 1000 more) and 129 us by tiles (flat up to ~8000 rows, a tile a CU).
-constexpr int64_t PRED_ROW_BLOCKS = 2048;
-// Rows from which tiles of 256 (each stages the forest once per 256 rows or
-// more) beat tiles of 64 (four times as many blocks): 20 000 rows 187 us by
-// 64, 65 536 rows 234 us by 256.
-constexpr int64_t PRED_WIDE_ROWS = 32768;
-
 // Staging a tile reads whole rows; the walks of a few trees touch only some of
-// a wide row's lines.  1M rows x 100 features, 1 / 2 trees of 63 leaves: 328 /
-// 342 us staged, 122 / 215 us not; 1M x 28, 1 tree: 62 against 120 us.
-inline bool stage_rows(int F, int T) { return F <= 28 * (T + 1); }
+// a wide row's lines.  1M rows x 100 features, 1 / 2 trees of 63 linear leaves: 328 /
+// 342 us staged, 122 / 215 us not; 200 000 x 200, 8 trees of 31 146 and 167.  Constant
+// leaves read less: there 146 and 119, 600 000 x 300, 16 trees 1089 and 489 us; 4000
+// rows x 200 29 and 32.
+constexpr int64_t PRED_STAGE_ROWS = 16384;
+inline bool stage_rows(const Forest& A, int64_t n) {
+    return A.F <= (A.net_k || n < PRED_STAGE_ROWS ? 28 : 16) * (A.T + 1);
+}
+
+// Few trees, whose walks cost less than a tile's fixed steps (about 4.5 us a tile and
+// CU).  One tree: with constant leaves always (1M rows x 28, 31 leaves: 74 us by
+// tiles, 63 by rows; x 10 73 and 41; 20 000 rows 28 and 22), with linear ones
+// while the rows are few (20 000 x 28: 29 and 24 us; 1M x 28: 73 and 114) or the
+// tree is larger than the LDS, but for rows that are little more than the walk
+// reads (1M x 300, 1000 leaves: 502 and 427; x 10 194 and 151; x 28 198 and 221).
+// Constant leaves: two trees, 1M x 10 75 and 60, 300 000 x 28 41 and 38, 1M x 28
+// 80 and 98 us; three on narrow rows, 300 000 x 10 42 and 39, of 1000 leaves 72
+// and 57; rows that are not staged, 200 000 x 100, 4 trees 74 and 69, 600 000 x 100
+// 161 and 191, x 300 295 and 223; 1M x 300, 5 trees 510 and 435 us.
+constexpr int64_t PRED_FLAT_INPUTS = 12'000'000;
+constexpr int64_t PRED_FLAT_ROWS = 131072;
+constexpr int PRED_NARROW = 16;                // features of a row within one 64-byte line
+inline bool predict_flat(const Forest& A, int64_t n, bool staged) {
+    const int64_t inputs = n * A.F;
+    const bool narrow = A.F <= PRED_NARROW;
+    if (A.T == 0) return true;
+    if (A.T == 1)
+        return !A.net_k || inputs < PRED_FLAT_INPUTS || (A.n_total > 1024 && (narrow || A.F > 4 * PRED_NARROW));
+    if (A.net_k) return false;
+    if (A.T == 2 && inputs < PRED_FLAT_INPUTS) return true;
+    if (n < PRED_FLAT_ROWS) return false;
+    if (A.T <= 3 && narrow) return true;
+    return !staged && A.T <= 5 && A.n_total <= 4096 && (A.F > 8 * PRED_NARROW || inputs < 5 * PRED_FLAT_INPUTS / 2);
+}
 
 int predict_tiles(const Forest& A, const float* X, int64_t ldx, int64_t n, float base, int accumulate, float* out,
                   hipStream_t stream) {
     constexpr size_t TREES = 40 * 1024;        // of the block's LDS at least this for the trees
     const auto fits = [&](int R) {
-        return stage_rows(A.F, A.T) && predict_lds(R, true, false, A.F, PRED_TILES, PRED_TB, 0, 0) + TREES <= PRED_LDS;
+        return stage_rows(A, n) && predict_lds(R, true, false, A.F, PRED_TILES, PRED_TB, 0, 0) + TREES <= PRED_LDS;
     };
+    if (predict_flat(A, n, fits(64))) {
+        auto flat = n < PRED_FLAT_ROWS || A.F > PRED_NARROW ? k_predict_flat<true> : k_predict_flat<false>;
+        flat<<<launch_grid(n, BB, 8192), BB, 0, stream>>>(A, X, ldx, n, base, accumulate, out);
+        return launch_status("yabt_predict launch");
+    }
     if (n >= PRED_WIDE_ROWS && fits(256))
         return launch_predict<256, 4, true>(A, X, ldx, n, base, accumulate, out, stream);
     if (fits(64)) return launch_predict<64, 16, true>(A, X, ldx, n, base, accumulate, out, stream);
