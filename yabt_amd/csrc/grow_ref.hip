@@ -400,12 +400,13 @@ constexpr int TPT = WT / RB;              // rows per thread per tile
 // grow.c:289; t0 % 16 == 0), 16 rows a thread with one load where every column
 // is 16-byte aligned and padded to 16 rows, else a row a load; by row id from
 // the row-major copy else.
-template <bool ROOT>
+enum BinsOf { CHILD, ROOT_VEC, ROOT_BYTES };
+template <BinsOf OF>
 __device__ __forceinline__ void tile_bins(const uint8_t* __restrict__ bins_fm, int64_t ld_fm,
                                           const uint8_t* __restrict__ bins_rm, int64_t ld_rm,
                                           const uint32_t* __restrict__ crow, int f, int64_t t0, int tn, uint8_t* s_bin) {
     const int tid = threadIdx.x;
-    if (ROOT && (((uintptr_t)bins_fm | (uintptr_t)ld_fm) & 15u) == 0) {
+    if (OF == ROOT_VEC) {
         static_assert(TPT == 16, "a thread's rows are one 16-byte load");
         if (tid * 16 < tn)
             *reinterpret_cast<uint4*>(s_bin + tid * 16) =
@@ -416,8 +417,8 @@ __device__ __forceinline__ void tile_bins(const uint8_t* __restrict__ bins_fm, i
     for (int j = 0; j < TPT; ++j) {
         const int x = j * RB + tid;
         if (x < tn)
-            s_bin[x] = ROOT ? bins_fm[(size_t)f * (size_t)ld_fm + (size_t)(t0 + x)]
-                            : bins_rm[(size_t)crow[t0 + x] * (size_t)ld_rm + f];
+            s_bin[x] = OF != CHILD ? bins_fm[(size_t)f * (size_t)ld_fm + (size_t)(t0 + x)]
+                                   : bins_rm[(size_t)crow[t0 + x] * (size_t)ld_rm + f];
     }
 }
 
@@ -430,7 +431,7 @@ __device__ __forceinline__ void tile_bins(const uint8_t* __restrict__ bins_fm, i
 // each lane's bit into s_peer[w][bin] (order-free), read back and cleared; a
 // row's rank is the number of those lanes below it plus the wave's running
 // count s_cnt[w][bin].
-template <bool ROOT>
+template <BinsOf OF>
 __global__ void __launch_bounds__(RB, 8) k_walk_sort(const uint8_t* __restrict__ bins_fm, int64_t ld_fm,
                                                      const uint8_t* __restrict__ bins_rm, int64_t ld_rm,
                                                      const uint32_t* __restrict__ rows, int64_t rows_ld,
@@ -457,7 +458,7 @@ __global__ void __launch_bounds__(RB, 8) k_walk_sort(const uint8_t* __restrict__
         (&s_cnt[0][0])[i] = 0;
         (&s_peer[0][0])[i] = 0;
     }
-    tile_bins<ROOT>(bins_fm, ld_fm, bins_rm, ld_rm, rows + (size_t)J.dst * (size_t)rows_ld + J.cs, f, t0, tn, s_bin);
+    tile_bins<OF>(bins_fm, ld_fm, bins_rm, ld_rm, rows + (size_t)J.dst * (size_t)rows_ld + J.cs, f, t0, tn, s_bin);
     __syncthreads();
     // per group: the rank (bits 0-9) and the bin (bits 24-31) in one register
     uint32_t pk[SGR];
@@ -525,7 +526,7 @@ __global__ void __launch_bounds__(RB, 8) k_walk_sort(const uint8_t* __restrict__
 // QUAD: block x takes the four features 4 x .. 4 x + 3 (those of the group), whose
 // bytes of a row it gathers with one 4-byte load: the gathers touch a row's
 // line once per four features (1.9 ms of child sorts a tree against 4.0).
-template <bool ROOT, bool QUAD>
+template <BinsOf OF, bool QUAD>
 __global__ void __launch_bounds__(RB, QUAD ? 3 : 5) k_walk_sort_sparse(const uint8_t* __restrict__ bins_fm, int64_t ld_fm,
                                                             const uint8_t* __restrict__ bins_rm, int64_t ld_rm,
                                                             const uint32_t* __restrict__ rows, int64_t rows_ld,
@@ -574,8 +575,7 @@ __global__ void __launch_bounds__(RB, QUAD ? 3 : 5) k_walk_sort_sparse(const uin
                 (&s_peer[0][0])[i] = 0;
             }
             if (!QUAD)
-                tile_bins<ROOT>(bins_fm, ld_fm, bins_rm, ld_rm, rows + (size_t)J.dst * (size_t)rows_ld + J.cs, f, t0, tn,
-                                s_bin);
+                tile_bins<OF>(bins_fm, ld_fm, bins_rm, ld_rm, rows + (size_t)J.dst * (size_t)rows_ld + J.cs, f, t0, tn, s_bin);
             __syncthreads();
             // thread tid: rows 16 tid ..; which of them are listed
             uint32_t bw[4];
@@ -2114,6 +2114,7 @@ struct Grower {
     // the sparse builder's arithmetic (grow.c:68-107).
     void hist(bool root, int K, int64_t tiles, const float* G, const float* H) {
         const unsigned ty = (unsigned)min((int64_t)65535, max((int64_t)1, tiles));
+        const bool vec = aligned16(bins_fm) && ld_fm % 16 == 0;
         for (int fg0 = 0; fg0 < F; fg0 += w.fgroup) {
             const int nf = min(w.fgroup, F - fg0);
             const dim3 sgrid((unsigned)nf, ty);
@@ -2121,14 +2122,14 @@ struct Grower {
                 // four features a block where that still fills the device
                 const int quads = (fg0 + nf - 1) / 4 - fg0 / 4 + 1;
                 const bool quad = !root && (int64_t)quads * tiles >= SORT_QUAD_BLOCKS;
-                auto sort = root ? k_walk_sort_sparse<true, false>
-                                 : (quad ? k_walk_sort_sparse<false, true> : k_walk_sort_sparse<false, false>);
+                auto sort = root ? (vec ? k_walk_sort_sparse<ROOT_VEC, false> : k_walk_sort_sparse<ROOT_BYTES, false>)
+                                 : (quad ? k_walk_sort_sparse<CHILD, true> : k_walk_sort_sparse<CHILD, false>);
                 sort<<<quad ? dim3((unsigned)quads, ty) : sgrid, RB, 0, st>>>(
                     bins_fm, ld_fm, bins_rm, ld_rm, w.rows, w.rows_ld, w.round, fg0, nf, dbin, w.perm, w.xperm, w.ld_perm,
                     w.starts, w.n_tiles);
                 if (fg0 == 0) k_total_tries<<<ty, RB, 0, st>>>(G, H, w.round, w.tries);
             } else {
-                auto sort = root ? k_walk_sort<true> : k_walk_sort<false>;
+                auto sort = !root ? k_walk_sort<CHILD> : vec ? k_walk_sort<ROOT_VEC> : k_walk_sort<ROOT_BYTES>;
                 sort<<<sgrid, RB, 0, st>>>(bins_fm, ld_fm, bins_rm, ld_rm, w.rows, w.rows_ld, w.round, fg0, w.perm,
                                            w.ld_perm, w.starts, w.n_tiles);
             }
