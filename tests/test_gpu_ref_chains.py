@@ -43,10 +43,15 @@ def test_root_histogram_at_tile_edges(n, F, top):
     (9_001, 4, 200, 16),     # rows in bins past the declared count: the last group's
     (5_003, 40, 64, 64),     # few groups, then (40 features x 16 jobs) k_walk_chain_dense
     (4_099, 600, 32, 32),    # k_walk_chain_dense from the root on
+    (70_001, 4, 256, 256),   # children of four tiles and more: k_tile_chain in 8 bin groups, later rounds dense
+    (70_003, 5, 200, 16),    # the same with rows past the declared count
+    (50_003, 70, 64, 64),    # two or three groups, then one block a feature
+    (36_001, 260, 40, 40),   # more features than CUs: dense, the root from the table too
 ])
 def test_bucketed_root_and_children(n, F, top, nb):
     """The root bucketed in the call and the root of the per-fit table take
-    different kernels or bin counts: same trees, bit for bit."""
+    different kernels or bin counts, and both trees are the oracle's, bit for
+    bit."""
     bins, g, h = _data(n, F, top)
     lay = G.make_layouts(torch.from_numpy(bins), DEV)
     kw = dict(fmask=None, imat=None, ib=0.0, lam=1.0, gamma=0.0, mcw=1e-3, msl=5, lr=0.1, max_leaves=63, max_depth=64)
@@ -59,10 +64,10 @@ def test_bucketed_root_and_children(n, F, top, nb):
     for name in ("feature", "thr_bin", "left", "right", "depth", "rows", "leaf_of_row"):
         assert torch.equal(getattr(a, name), getattr(b, name)), name
     assert torch.equal(a.value.view(torch.int32), b.value.view(torch.int32))
-    if nb == top:
-        want = O.grow(np.ascontiguousarray(bins.T), g, h, mode=O.MODE_FP32, nbins=nbins, msl=5, max_leaves=63)
-        assert np.array_equal(a.feature.cpu().numpy(), want["feature"])
-        assert np.array_equal(a.value.cpu().numpy().view(np.uint32), want["value"].view(np.uint32))
+    want = O.grow(np.ascontiguousarray(bins.T), g, h, mode=O.MODE_FP32, nbins=nbins, msl=5, max_leaves=63)
+    got = {k: getattr(a, k).cpu().numpy() for k in ("feature", "thr_bin", "left", "right", "value", "depth")}
+    assert tree_arrays_equal(got, want) is None
+    assert np.array_equal(a.rows.cpu().numpy(), want["rows"])
 
 
 @pytest.mark.parametrize("sparse", [False, True])

@@ -5,10 +5,10 @@
 // except where cgrow's own fp32 rounding decides a split.  This grower
 // reproduces cgrow's arithmetic instead:
 //   * a node histogram is the fp32 sum, per (feature, bin), of the node's rows
-//     in the order cgrow's rows[] array holds them (grow.c:37-62): one block
-//     per feature streams the node's rows in that order, buckets each tile by
-//     bin with a stable counting sort in LDS, and one thread per bin keeps the
-//     bin's running sums (the sparse builder, grow.c:68-107, likewise);
+//     in the order cgrow's rows[] array holds them (grow.c:37-62): each tile
+//     of the node's rows in that order is bucketed by bin with a stable counting
+//     sort in LDS, all tiles at once, and one thread per bin and channel adds
+//     the bin's runs tile by tile (the sparse builder, grow.c:68-107, likewise);
 //   * rows[] follows cgrow's in-place two-pointer partition (grow.c:201-217),
 //     which is a fixed permutation of the node's rows, computed in parallel
 //     (see "partition" below);
@@ -378,13 +378,14 @@ __global__ void __launch_bounds__(RB) k_part_permute(const uint8_t* __restrict__
 // parallel over the whole device; a chain kernel then runs one block per
 // (feature, split) over the tiles in order, adding bin b's run of each tile
 // to its fp32 accumulators, so every cell is cgrow's sequential sum.
-// Dense (k_tile_chain, k_walk_chain_dense): the tile's g and h permuted into bucket order
-// in LDS, one thread per (bin, channel).
+// Dense (k_tile_chain, k_walk_chain_dense): the tile's g and h permuted into
+// bucket order in LDS, one thread per (bin, channel); k_tile_chain spreads a
+// feature's bins over several blocks where features are few.
 //
 // Sparse builder (grow.c:68-107, default bins dbin; k_walk_chain_sparse): the
-// default bin gets no run; its thread instead adds, in double and in row
-// order, the tile's rows outside the default bin; block F adds the node's g
-// and h in double in row order; k_hist_default combines them.
+// default bin gets no run; two waves add, in double and in row order, the
+// tile's rows outside the default bin (g and h); one more block adds the
+// node's g and h in double in row order; k_hist_default combines them.
 
 constexpr int SW = RB / WAVE;             // waves per sort / chain block
 // Blocks of a sparse sort that fill the device (3 a CU, twice over and more):
@@ -1306,23 +1307,30 @@ __device__ __forceinline__ void dense_load(DenseTile& c, const float* __restrict
 // the tile's pairs permuted into bucket order in LDS (channel by channel,
 // so a bin's run is contiguous); the count cell is cgrow's chain of 1.0f
 // adds, min(count, 2^24).  A bin's two channels run in different waves:
-// one dependent add per row and thread.
+// one dependent add per row and thread.  ROOT: the node is every row, as
+// k_tile_chain's.
+template <bool ROOT>
 __global__ void __launch_bounds__(CB) k_walk_chain_dense(const float* __restrict__ Gb, const float* __restrict__ Hb,
-                                                         const Round* __restrict__ R, int F, int fg0,
+                                                         int64_t n, const Round* __restrict__ R, int F, int fg0,
                                                          const uint16_t* __restrict__ perm, int64_t ld_perm,
                                                          const uint16_t* __restrict__ starts, int64_t n_tiles,
                                                          float* __restrict__ hist_base, size_t hsz) {
     __shared__ __align__(16) float2 s_gh[WT];
     __shared__ float s_ch[2][WT];    // g, h in bucket order
     __shared__ uint16_t s_st[ST];
-    const int kj = blockIdx.y;
-    const Job& J = R->job[kj];
-    const int64_t m = J.ce - J.cs;
-    const int64_t tile0 = R->toff[kj];
-    const float* G = Gb + J.cs;
-    const float* H = Hb + J.cs;
     const int tid = threadIdx.x, ch = tid / NB, b = tid % NB;
     const int fl = blockIdx.x, f = fg0 + fl;       // buffers by group position, cells by feature
+    int64_t m = n, tile0 = 0;
+    const float *G = Gb, *H = Hb;
+    float* hist = hist_base;
+    if (!ROOT) {
+        const Job& J = R->job[blockIdx.y];
+        m = J.ce - J.cs;
+        tile0 = R->toff[blockIdx.y];
+        G += J.cs;
+        H += J.cs;
+        hist += (size_t)(J.build_left ? J.slot_l : J.slot_r) * hsz;
+    }
     const uint16_t* pf = perm + (size_t)fl * (size_t)ld_perm + (size_t)tile0 * WT;
     const uint16_t* sf = starts + ((size_t)fl * (size_t)n_tiles + (size_t)tile0) * ST;
     float acc = 0.0f;
@@ -1358,8 +1366,6 @@ __global__ void __launch_bounds__(CB) k_walk_chain_dense(const float* __restrict
         cnt += hi - lo;
         __syncthreads();
     }
-    const int slot = J.build_left ? J.slot_l : J.slot_r;
-    float* hist = hist_base + (size_t)slot * hsz;
     hist[(size_t)ch * F * NB + (size_t)f * NB + b] = acc;
     if (ch == 0) hist[(size_t)2 * F * NB + (size_t)f * NB + b] = (float)min(cnt, (int64_t)1 << 24);
 }
@@ -1401,14 +1407,21 @@ constexpr int CPAD = 8 * CDEEP;      // cells run_f32 may read past a tile
 
 // Bin groups per feature of a k_tile_chain launch: blocks for one a CU (every
 // group's block loads the whole tile, so more groups only repeat loads).  0
-// where features and jobs alone are more than two blocks a CU: there the
-// chains are bound by the device's throughput, and k_walk_chain_dense's
-// smaller blocks take less (1M x 100, 16 jobs a round, late rounds: 30 against
-// 34 us; 300 features, 16 jobs: a 30 000-row tree 1.25 against 1.55 ms).
+// where k_walk_chain_dense, which keeps two blocks on a CU, is the faster: the
+// root from more than one block a CU (300 000 x 300 at 16, 64 and 256 bins 333,
+// 244 and 236 against 396, 279 and 269 us); the children of more than two (300
+// features, 16 jobs: a 30 000-row tree 1.25 against 1.55 ms), where the chains are
+// bound by the device's throughput (between one and two k_tile_chain's longer runs
+// of few bins gain: 28 features, 16 jobs of a 1M-row tree 66 us a launch, 71),
+// and of jobs of few tiles, since a job's first tile is added in its third step
+// on average (30 features, 1.5: 4, 8 and 16 jobs 5.2, 4.2 and 4.3 us against
+// 6.1, 6.6 and 10.6; one job of 4 tiles 9.6 and 8.1).
 constexpr int CHAIN_BLOCKS = 256;
-inline int chain_groups(int nf, int jobs) {
+constexpr int CHAIN_TILES = 2;
+inline int root_groups(int F) { return F > CHAIN_BLOCKS ? 0 : min(8, CHAIN_BLOCKS / F); }
+inline int chain_groups(int nf, int jobs, int64_t tiles) {
     const int64_t blocks = (int64_t)nf * jobs;
-    if (blocks > 2 * CHAIN_BLOCKS) return 0;
+    if (blocks > 2 * CHAIN_BLOCKS || tiles < (int64_t)CHAIN_TILES * jobs) return 0;
     return (int)min((int64_t)8, max((int64_t)1, CHAIN_BLOCKS / blocks));
 }
 
@@ -1449,9 +1462,12 @@ static_assert(CPT * sizeof(uint16_t) == sizeof(Pos8), "a thread's list entries a
 // largest bins give the bin count); else job blockIdx.y's built child.
 // What bounds it: the dependent adds (~15 cycles a row of the longest bin, LDS
 // reads included) at few bins, the loading threads' LDS passes (~0.8 us a tile)
-// at 256.  One block per feature and 256 adding threads took 1106 us for the
-// root of 1M x 28 at 28 bins and 312 at 256 bins; now 406 and 220 (10M x 100:
-// 3.05 -> 3.06 ms), the children of that tree 1671 -> 1300 us.  Waves that each
+// at 256.  One block per feature and 256 adding threads, from a table of ranks,
+// took 1106 us for the root of 1M x 28 at 28 bins and 312 at 256 bins; now 406
+// and 220 (10M x 100: 3.05 -> 3.06 ms), the children of that tree 1671 -> 1300
+// us.  A block that has all of a feature's bins (129 to 256 features) is bound by
+// those passes: the root of 300 000 x 200 took 357, 175 and 122 us at 28, 100 and
+// 256 bins, now 174, 139 and 138.  Waves that each
 // gathered their own bins' g and h from L2 with no barrier took 447 us and, at
 // 10M x 100, 10.8 ms: a 4-byte gather moves a whole line.
 template <bool ROOT>
@@ -1530,8 +1546,10 @@ __global__ void __launch_bounds__(2 * CB) k_tile_chain(const float* __restrict__
                 bounds(k, t + 2);
                 if (__any(len > 64u))
                     run_f32<CDEEP>(s_ch[k][ch] + at, len, acc);
-                else if (__any(len > 0u))
+                else if (__any(len > 32u))
                     run_f32<2>(s_ch[k][ch] + at, len, acc);
+                else if (__any(len > 0u))
+                    run_f32<1>(s_ch[k][ch] + at, len, acc);
                 cnt += len;
                 __syncthreads();
             }
@@ -1737,8 +1755,13 @@ __global__ void __launch_bounds__(RB, 8) k_root_order(const uint8_t* __restrict_
 
 inline void launch_root_chain(const float* g, const float* h, int64_t n, const RootOrder& o, float* hist, int F,
                               hipStream_t stream) {
-    k_tile_chain<true><<<(unsigned)(F * max(1, chain_groups(F, 1))), 2 * CB, 0, stream>>>(
-        g, h, n, nullptr, F, 0, F, o.perm, o.ld_perm, o.starts, o.tiles, nullptr, o.maxbin, hist, 0);
+    const int groups = root_groups(F);
+    if (groups > 0)
+        k_tile_chain<true><<<(unsigned)(F * groups), 2 * CB, 0, stream>>>(
+            g, h, n, nullptr, F, 0, F, o.perm, o.ld_perm, o.starts, o.tiles, nullptr, o.maxbin, hist, 0);
+    else
+        k_walk_chain_dense<true><<<(unsigned)F, CB, 0, stream>>>(g, h, n, nullptr, F, 0, o.perm, o.ld_perm, o.starts, o.tiles,
+                                                                 hist, 0);
 }
 
 // Sparse builder's default-bin cells (grow.c:101-106): 0 + (float)(node sum -
@@ -2138,12 +2161,12 @@ struct Grower {
             if (dbin)
                 k_walk_chain_sparse<<<cgrid, RB, 0, st>>>(G, H, w.round, F, fg0, nf, dbin, w.perm, w.xperm, w.ld_perm,
                                                           w.starts, w.n_tiles, w.hist, hsz, w.tries, w.expl, w.tot);
-            else if (chain_groups(nf, K) > 0)
-                k_tile_chain<false><<<dim3((unsigned)(nf * chain_groups(nf, K)), (unsigned)K), 2 * CB, 0, st>>>(
+            else if (const int groups = chain_groups(nf, K, tiles))
+                k_tile_chain<false><<<dim3((unsigned)(nf * groups), (unsigned)K), 2 * CB, 0, st>>>(
                     G, H, n, w.round, F, fg0, nf, w.perm, w.ld_perm, w.starts, w.n_tiles, nbins, nullptr, w.hist, hsz);
             else
-                k_walk_chain_dense<<<cgrid, CB, 0, st>>>(G, H, w.round, F, fg0, w.perm, w.ld_perm, w.starts,
-                                                         w.n_tiles, w.hist, hsz);
+                k_walk_chain_dense<false><<<cgrid, CB, 0, st>>>(G, H, n, w.round, F, fg0, w.perm, w.ld_perm, w.starts,
+                                                                w.n_tiles, w.hist, hsz);
         }
         if (dbin)
             k_hist_default<<<dim3((F + RB - 1) / RB, (unsigned)K), RB, 0, st>>>(dbin, w.expl, w.tot, F, w.hist, hsz,
