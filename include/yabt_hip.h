@@ -400,8 +400,8 @@ size_t yabt_ref_root_order_bytes(int64_t n, int F);
 
 /* The root table of yabt_grow_ref's dense builder, once per fit: for
  * every feature and every 4096-row tile of rows 0 .. n - 1, the tile's rows
- * bucketed by bin (row order inside a bin), the tile's bin starts, its
- * longest run and its largest bin --
+ * bucketed by bin (row order inside a bin), the tile's bin starts and its
+ * largest bin --
  * the bucketing of cgrow's row-order histogram chains (yabt/_cgrow/grow.c:
  * 37-62) of the root, which is the same for every tree grown on these bins.
  * out: device memory of at least yabt_ref_root_order_bytes(n, F) bytes.
@@ -414,7 +414,8 @@ int yabt_ref_root_order(const uint8_t *bins_fm, int64_t ld_fm, int64_t n, int F,
  * cgrow's dense build_hist over rows 0 .. n - 1 (yabt/_cgrow/grow.c:37-62):
  * per (feature, bin) the fp32 sums of g, of h and of 1.0f in row order, from
  * the root table yabt_ref_root_order made for these bins (root_order_bytes:
- * its size).  Replaces build_hist for the root node. */
+ * its size); bins_fm is not read, but must be given.  Replaces build_hist for
+ * the root node. */
 int yabt_ref_root_hist(const uint8_t *bins_fm, int64_t ld_fm, const float *grad, const float *hess, int64_t n,
                        int F, const void *root_order, size_t root_order_bytes, float *out, yabt_stream_t stream);
 

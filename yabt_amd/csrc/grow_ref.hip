@@ -1635,12 +1635,11 @@ __global__ void __launch_bounds__(2 * CB) k_tile_chain(const float* __restrict__
 
 // The root table of yabt_ref_root_order: each tile's positions bucketed by bin
 // (uint16, F x ld_perm), the run starts (uint16, F x tiles x ST, as
-// k_walk_sort's), each (feature, tile)'s longest run (uint16, F x tiles) and
-// its largest bin present (uint8, F x tiles).
+// k_walk_sort's) and each (feature, tile)'s largest bin present (uint8, F x
+// tiles).
 struct RootOrder {
     uint16_t* perm;
     uint16_t* starts;
-    uint16_t* maxrun;
     uint8_t* maxbin;
     int64_t ld_perm;
     int64_t tiles;
@@ -1651,17 +1650,15 @@ __host__ __device__ inline size_t root_order_carve(char* base, int64_t n, int F,
     const int64_t ld = tiles * WT;
     const size_t perm_bytes = ((size_t)F * (size_t)ld * sizeof(uint16_t) + 255) / 256 * 256;
     const size_t st_bytes = ((size_t)F * (size_t)tiles * ST * sizeof(uint16_t) + 255) / 256 * 256;
-    const size_t mx_bytes = ((size_t)F * (size_t)tiles * sizeof(uint16_t) + 255) / 256 * 256;
     const size_t mb_bytes = ((size_t)F * (size_t)tiles + 255) / 256 * 256;
     if (o) {
         o->perm = (uint16_t*)base;
         o->starts = (uint16_t*)(base + perm_bytes);
-        o->maxrun = (uint16_t*)(base + perm_bytes + st_bytes);
-        o->maxbin = (uint8_t*)(base + perm_bytes + st_bytes + mx_bytes);
+        o->maxbin = (uint8_t*)(base + perm_bytes + st_bytes);
         o->ld_perm = ld;
         o->tiles = tiles;
     }
-    return perm_bytes + st_bytes + mx_bytes + mb_bytes;
+    return perm_bytes + st_bytes + mb_bytes;
 }
 
 // Block (f, t): feature f's tile t bucketed as in k_walk_sort (tiles grid-
@@ -1672,7 +1669,7 @@ __global__ void __launch_bounds__(RB, 8) k_root_order(const uint8_t* __restrict_
     __shared__ uint64_t s_peer[SW][NB];            // once the tile is ranked: its bucketed positions
     __shared__ uint32_t s_cnt[SW][NB];
     __shared__ uint32_t s_scan[SW];
-    __shared__ uint32_t s_max, s_mb;
+    __shared__ uint32_t s_mb;
     uint16_t* s_perm = reinterpret_cast<uint16_t*>(&s_peer[0][0]);
     const int f = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
@@ -1683,10 +1680,7 @@ __global__ void __launch_bounds__(RB, 8) k_root_order(const uint8_t* __restrict_
             (&s_cnt[0][0])[i] = 0;
             (&s_peer[0][0])[i] = 0;
         }
-        if (tid == 0) {
-            s_max = 0;
-            s_mb = 0;
-        }
+        if (tid == 0) s_mb = 0;
 #pragma unroll
         for (int j = 0; j < TPT; ++j) {
             const int x = j * RB + tid;
@@ -1722,13 +1716,9 @@ __global__ void __launch_bounds__(RB, 8) k_root_order(const uint8_t* __restrict_
                 tb += c[u];
             }
             uint32_t total;
-            atomicMax(&s_max, tb);
             if (tb) atomicMax(&s_mb, (uint32_t)b);
             const uint32_t st = block_excl_scan<RB, uint32_t>(tb, s_scan, &total);
-            if (tid == 0) {
-                o.maxrun[(size_t)f * (size_t)o.tiles + (size_t)t] = (uint16_t)s_max;
-                o.maxbin[(size_t)f * (size_t)o.tiles + (size_t)t] = (uint8_t)s_mb;
-            }
+            if (tid == 0) o.maxbin[(size_t)f * (size_t)o.tiles + (size_t)t] = (uint8_t)s_mb;
             uint16_t* st_out = o.starts + ((size_t)f * (size_t)o.tiles + (size_t)t) * ST;
             st_out[b] = (uint16_t)st;
             if (b == NB - 1) st_out[NB] = (uint16_t)(st + tb);
