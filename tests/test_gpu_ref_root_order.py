@@ -1,14 +1,10 @@
-"""The reference-arithmetic grower's per-fit root rank table
-(yabt_ref_root_order + k_rank_chain) against the per-tree bucketing of the
-root (k_walk_sort + k_walk_chain): identical trees, rows[] and leaf ids, bit
-for bit, on ragged tiles, a single partial tile, bins skewed enough that a
-tile's run of one bin exceeds both the chain's 32-rank LDS window and 255,
-and features of few bins (the window widened to 128 .. 4096 ranks).
-
-Both paths restate cgrow's row-order fp32 histogram chains
-(yabt/_cgrow/grow.c:37-62); their agreement with grow.c itself is checked by
-tests/test_gpu_grow_ref.py and tests/test_gpu_full_size.py, which grow through
-the rank table now.
+"""The reference-arithmetic grower's per-fit root table (yabt_ref_root_order)
+against the bucketing of the root in each call (k_walk_sort): identical trees,
+rows[] and leaf ids, bit for bit, and both the oracle's (its row-order fp32
+chains, oracle/grow_oracle.c; yabt/_cgrow/grow.c:37-62).  Ragged tiles, a single
+partial tile, runs of a bin that are longer than the chains' reads ahead (64, and
+most of a tile), and features of few bins, whose groups of bins differ between the
+two roots: the table knows the largest bin, the call only the declared count.
 """
 
 import numpy as np
@@ -26,11 +22,10 @@ def _bins(kind, n, F, rng):
     if kind == "uniform":
         return rng.integers(0, 256, size=(n, F)).astype(np.uint8)
     if kind == "few":
-        # per feature a different span of bins: 28 (a window of 256 ranks),
-        # 2, 1 (all zero: a window of the whole tile), 33 (bins 0..31 and a
-        # single row of bin 32 in one tile: a window of 128 ranks for every
-        # tile), 32, and 20 with 90% of rows in bin 3 (runs of ~3700 per tile,
-        # past the 256-rank window)
+        # per feature a different span of bins: 28, 2, 1 (all zero: one run of
+        # the whole tile, one group), 33 (bins 0..31 and a single row of bin 32
+        # in one tile, which the groups must cover), 32, and 20 with 90% of
+        # rows in bin 3 (runs of ~3700 per tile)
         spans = [28, 2, 1, 32, 32, 20]
         b = np.stack([rng.integers(0, spans[f % len(spans)], size=n) for f in range(F)], axis=1)
         sk = [f for f in range(F) if f % len(spans) == len(spans) - 1]
@@ -47,15 +42,17 @@ def _bins(kind, n, F, rng):
 @pytest.mark.parametrize("kind,n,F,leaves", [
     ("uniform", 50_000, 12, 31),     # 13 tiles, the last one partial
     ("uniform", 100, 5, 8),          # one partial tile
-    ("skewed", 30_000, 6, 24),       # runs longer than 32 and than 255 ranks
-    ("few", 60_000, 6, 31),          # spans of 1..33 bins: windows of 256..4096 ranks
+    ("skewed", 30_000, 6, 24),       # runs above and below 64
+    ("few", 60_000, 6, 31),          # spans of 1..33 bins: groups of 1 to 5 bins
 ])
 def test_rank_table_root_equals_bucketed_root(kind, n, F, leaves):
+    from oracle import oracle as O
+    from tests.helpers import tree_arrays_equal
     rng = np.random.default_rng(11)
     bins = _bins(kind, n, F, rng)
     lay = G.make_layouts(torch.from_numpy(bins), DEV)
-    g = torch.from_numpy(rng.normal(size=n).astype(np.float32)).to(DEV)
-    h = torch.from_numpy(rng.uniform(0.05, 1.0, size=n).astype(np.float32)).to(DEV)
+    gh = rng.normal(size=n).astype(np.float32), rng.uniform(0.05, 1.0, size=n).astype(np.float32)
+    g, h = (torch.from_numpy(v).to(DEV) for v in gh)
     nbins = np.full(F, 256, np.int32)
     kw = dict(fmask=None, imat=None, ib=0.0, lam=1.0, gamma=0.0, mcw=1e-3, msl=5, lr=0.1,
               max_leaves=leaves, max_depth=64)
@@ -69,6 +66,10 @@ def test_rank_table_root_equals_bucketed_root(kind, n, F, leaves):
     assert torch.equal(a.value.view(torch.int32), b.value.view(torch.int32))
     assert torch.equal(a.rows, b.rows)
     assert torch.equal(a.leaf_of_row, b.leaf_of_row)
+    want = O.grow(np.ascontiguousarray(bins.T), *gh, mode=O.MODE_FP32, nbins=nbins, msl=5, max_leaves=leaves)
+    got = {k: getattr(a, k).cpu().numpy() for k in ("feature", "thr_bin", "left", "right", "value", "depth")}
+    assert tree_arrays_equal(got, want) is None
+    assert np.array_equal(a.rows.cpu().numpy(), want["rows"])
 
 
 @pytest.mark.parametrize("kind,n,F", [("uniform", 70_001, 9), ("skewed", 20_000, 4), ("few", 50_003, 12)])
