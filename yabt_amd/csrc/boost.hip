@@ -232,11 +232,12 @@ __global__ void __launch_bounds__(BB) k_predict_flat(Forest A, const float* __re
 // 500 000 rows x 50 features, 200 trees of 63 leaves with 8 inputs: 1.41 ms
 // (0.63 ms without linear leaves), 18.9 ms by a walk per row and tree in
 // global memory, which waited on a gather of 32 node bytes and one of the
-// row's input per level.  Counters: LDS active 40% and VALU 42% of the time,
-// the rest latency at the 16 waves a CU that the tile's LDS leaves (a longer
-// list of walks per thread in one loop, lanes going on by themselves: 2.2 ms;
-// the end's select and its own slot per step: 1.75 ms; inputs not loaded
-// ahead, batches not a multiple of the groups: 1.52 ms).
+// row's input per level.  Counters: LDS active 49% and VALU 44% of the time,
+// bank conflicts 17%; a wave waits 48% of its time, and the tile's LDS leaves
+// no more than 16 waves a CU to cover that (a longer list of walks per thread in
+// one loop, lanes going on by themselves: 2.2 ms; the end's select and its own
+// slot per step: 1.75 ms; inputs not loaded ahead, batches not a multiple of the
+// groups: 1.52 ms).
 constexpr int PRED_TB = 32;                    // trees per batch at most
 constexpr int PRED_TILES = 16;                 // tiles per block at most
 constexpr int PRED_LEAF = 28;                  // floats per leaf: 8 weights, 8 lows, 8 highs, value, padding
@@ -498,13 +499,17 @@ size_t predict_lds(int R, bool xlds, bool lin, int F, int tiles, int tb, int nca
 
 constexpr size_t PRED_LDS = 156 * 1024;        // dynamic LDS of a tile block (one a CU)
 
-// Rows up to which a block per row is faster than tiles of rows: with 200
-// trees of 63 linear leaves, 50 features, 2048 rows take 94 us by blocks (46 us
-// per 1000 more) and 129 us by tiles (flat up to ~8000 rows, a tile a CU).
+// Rows up to which a block per row takes less than tiles of rows.  By rows and by
+// tiles, us: 200 trees of 63 linear leaves, 50 features, 2048 rows 110 and 140, 3000
+// 150 and 140; 10 of 31, 28 features 26 and 27, 30 and 27; 1000 of 20 constant
+// leaves 186 and 224, 263 and 224; 40 of 31 24 and 32, at 6000 rows 33 and 33; 30 of
+// 255 linear leaves 33 and 60, at 6000 58 and 57.
 constexpr int64_t PRED_ROW_BLOCKS = 2048;
-// Rows from which tiles of 256 (each stages the forest once per 256 rows or
-// more) beat tiles of 64 (four times as many blocks): 20 000 rows 187 us by
-// 64, 65 536 rows 234 us by 256.
+// Rows from which tiles of 256 (each stages the forest once per 256 rows or more)
+// beat tiles of 64 (four times as many blocks).  By 64 and by 256, us: 200 trees of
+// 63 linear leaves, 50 features, 20 000 rows 191 and 227, 32 768 194 and 230, 40 000
+// 242 and 233, 65 536 301 and 244; 30 of 255 101 and 122, 123 and 121, 158 and 122;
+// 200 of 63 constant leaves 116 and 105, 117 and 105, 150 and 105.
 constexpr int64_t PRED_WIDE_ROWS = 32768;
 
 // Tiles of a block: one block a CU, in as many rounds of them as PRED_TILES asks,
